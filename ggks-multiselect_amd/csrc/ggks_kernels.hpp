@@ -16,9 +16,11 @@
 //             into its private slice of the child's range
 //   k_finish_small  per child with few ranks: top-digit histogram, then the
 //             rank's digit gathered and ranked (keys in registers when they
-//             fit); per child of up to 1024 keys with many ranks: LDS sort
-//   k_finish  every other child: multi-rank MSD radix select on 8-bit digits
-//             of (key - lo), or a sort, keys resident in LDS when they fit
+//             fit); per child of up to 1024 keys with many ranks: its keys
+//             in LDS in the order of nearly even bins (bin_select)
+//   k_finish  every other child: bin_select when its keys fit LDS (a sort or
+//             8-bit digit passes where bins stay crowded), else multi-rank
+//             MSD radix select on 8-bit digits of (key - lo) from memory
 // Plans of at most 4096 buckets per segment run k_findk_small and
 // k_compact_small: the same bodies with smaller tables, two work-groups per
 // CU.  Plans whose children are small run k_finish_small_lite (4-byte keys):
@@ -91,6 +93,18 @@ __device__ __forceinline__ void lds_or(uint32_t* w, uint32_t idx, uint32_t v) {
 // Value of lane 63 (the wavefront total after an inclusive scan), uniform.
 __device__ __forceinline__ uint32_t wave_last(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Lane l's value (l uniform).
+template <typename KT>
+__device__ __forceinline__ KT wave_lane(KT v, uint32_t l) {
+  if constexpr (sizeof(KT) == 4) {
+    return (KT)__builtin_amdgcn_readlane((int)v, (int)l);
+  } else {
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)l);
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)l);
+    return (KT)(((uint64_t)b << 32) | a);
+  }
 }
 
 // Block-wide exclusive scan of one value per thread (blockDim.x == 1024).
@@ -2451,6 +2465,247 @@ __device__ __forceinline__ void wave_pick256(const uint32_t* h, uint32_t lane, u
   below = (uint32_t)__shfl((int)start, src, 64);
 }
 
+// Many ranks of one child whose keys a work-group of NT threads holds in
+// registers (S a thread, so at most S * NT keys): the keys are scattered into
+// LDS in the order of FB nearly even bins, and every rank is then among the
+// few keys of the bin that position rank - 1 falls in.  Two histograms, two
+// scans and one scatter, eight barriers, whatever the number of ranks.
+//   bins    NT coarse bins split the keys' own range (the first and last
+//           bucket of a segment reach to the ends of the key space) evenly,
+//           and each coarse bin takes fine bins in proportion to its keys:
+//           with even bins alone a normal's tail or the keys around zero (a
+//           whole vector of floats, too) crowd into a few of them.
+//   a rank  in a bin of one key: that key.  Up to kBinThread keys: one thread
+//           counts them against each other.  Up to 64: a wavefront does, a
+//           key a lane.  More: 8-bit digits by one wavefront over the bin.
+// Bound by its LDS round trips and barriers.  Against the digit passes and
+// sorts of whole children that it replaced (k_finish, start to end): 10 007
+// keys, 16 ranks 34.5 -> 10.5 us; the 4096 largest of 2^28 in two children of
+// 5602 and 2880 keys 48 -> 18 us; 256 ranks in 1341 keys, ten copies a value,
+// 21 -> 14 us; a 4096-segment batch's children 472 -> 190 us.
+// Returns false (nothing lost: srt then holds the keys minus lo, in some
+// order) where the ranks of crowded bins would read more than kBinWork keys
+// in all; the caller then sorts or takes digit passes over the whole child.
+constexpr uint32_t kBinThread = 8;
+constexpr uint32_t kBinWork = 1u << 16;
+template <uint32_t NT>
+constexpr uint32_t kFineBins = NT == kThreads ? 8192 : 4 * NT;
+template <typename KT, int C, uint32_t NT, uint32_t S>
+__device__ bool bin_select(const KT* __restrict__ srcp, uint32_t len, const Query* __restrict__ cq,
+                           uint32_t q_cnt, KT* __restrict__ out, KT* srt, uint32_t* hist,
+                           uint32_t* coarse, uint32_t* whist, uint4* list, KT* red_lo, KT* red_hi,
+                           uint32_t* misc, KT& lo_out, int& nbits_out) {
+  constexpr uint32_t NW = NT / 64, FB = kFineBins<NT>, WPT = FB / NT;  // fine bins per thread
+  constexpr int BB = NT == 1024 ? 10 : 8;                              // log2 coarse bins
+  static_assert(NT == (1u << BB) && WPT % 4 == 0 && S * NT <= 32768, "bins");
+  const uint32_t tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+  // misc: NW wavefront totals, then the list's length and its keys
+  uint32_t* const wtot = misc;
+  uint32_t& nlist = misc[NW];
+  uint32_t& work = misc[NW + 1];
+  KT k[S];
+#pragma unroll
+  for (uint32_t t = 0; t < S; ++t) {
+    const uint32_t i = t * NT + tid;
+    k[t] = i < len ? srcp[i] : KT(0);
+  }
+  const Query q0 = tid < q_cnt ? cq[tid] : Query{1, 0};  // arrives with the keys
+#pragma unroll
+  for (uint32_t j = 0; j < WPT / 4; ++j)
+    reinterpret_cast<uint4*>(hist)[j * NT + tid] = make_uint4(0, 0, 0, 0);
+  coarse[tid] = 0;
+  if (tid == 0) {
+    nlist = 0;
+    work = 0;
+  }
+  KT a = KeyBits<KT>::MAX, b = 0;
+#pragma unroll
+  for (uint32_t t = 0; t < S; ++t) {
+    if (t * NT + tid < len) {
+      k[t] = to_key<C>(k[t]);
+      a = k[t] < a ? k[t] : a;
+      b = k[t] > b ? k[t] : b;
+    }
+  }
+  for (int d = 32; d >= 1; d >>= 1) {
+    const KT x = __shfl_xor(a, d, 64), y = __shfl_xor(b, d, 64);
+    a = x < a ? x : a;
+    b = y > b ? y : b;
+  }
+  if (lane == 0) {
+    red_lo[w] = a;
+    red_hi[w] = b;
+  }
+  __syncthreads();  // range parts, cleared bins
+  KT lo = red_lo[0], hi = red_hi[0];
+  for (uint32_t v = 1; v < NW; ++v) {
+    lo = red_lo[v] < lo ? red_lo[v] : lo;
+    hi = red_hi[v] > hi ? red_hi[v] : hi;
+  }
+  const int nbits = bitlen<KT>((KT)(hi - lo));
+  const int sh = nbits > BB ? nbits - BB : 0;
+#pragma unroll
+  for (uint32_t t = 0; t < S; ++t) {
+    if (t * NT + tid < len) {
+      k[t] -= lo;
+      atomicAdd(&coarse[(uint32_t)(k[t] >> sh)], 1u);
+    }
+  }
+  // exclusive prefix of v over the work-group's threads (two barriers, the
+  // second by the caller once it has stored what it derives)
+  auto prefix = [&](uint32_t v) {
+    const uint32_t inc = wave_incl_scan(v);
+    if (lane == 63) wtot[w] = inc;
+    __syncthreads();
+    const uint32_t ws = lane < NW ? wtot[lane] : 0u;
+    const uint32_t wi = wave_incl_scan(ws);
+    return (uint32_t)__builtin_amdgcn_readlane((int)(wi - ws), (int)w) + inc - v;
+  };
+  __syncthreads();  // coarse counts
+  {
+    // fine bins of this thread's coarse bin: in all at most FB
+    const uint32_t c = coarse[tid];
+    const uint32_t nb = c == 0 ? 0u : sh == 0 ? 1u : 1u + c * (FB - NT) / len;  // c (FB - NT) < 2^28
+    const uint32_t base = prefix(nb);
+    coarse[tid] = base | (nb << 16);
+  }
+  __syncthreads();  // coarse entries
+  uint32_t bp[S];  // a key's fine bin, and its place in it
+#pragma unroll
+  for (uint32_t t = 0; t < S; ++t) {
+    if (t * NT + tid < len) {
+      const uint32_t e = coarse[(uint32_t)(k[t] >> sh)];
+      // the bits below the coarse digit, from the top of a word
+      const uint32_t low = sh == 0 ? 0u : sh <= 32 ? (uint32_t)k[t] << (32 - sh) : (uint32_t)(k[t] >> (sh - 32));
+      const uint32_t bn = (e & 0xFFFFu) + __umulhi(low, e >> 16);
+      bp[t] = (bn << 16) | atomicAdd(&hist[bn], 1u);
+    }
+  }
+  __syncthreads();  // counts
+  {
+    uint32_t c[WPT], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < WPT / 4; ++j) {
+      const uint4 h4 = reinterpret_cast<const uint4*>(hist)[tid * (WPT / 4) + j];
+      c[4 * j] = sum; sum += h4.x;
+      c[4 * j + 1] = sum; sum += h4.y;
+      c[4 * j + 2] = sum; sum += h4.z;
+      c[4 * j + 3] = sum; sum += h4.w;
+    }
+    const uint32_t e = prefix(sum);
+#pragma unroll
+    for (uint32_t j = 0; j < WPT / 4; ++j)
+      reinterpret_cast<uint4*>(hist)[tid * (WPT / 4) + j] =
+          make_uint4(e + c[4 * j], e + c[4 * j + 1], e + c[4 * j + 2], e + c[4 * j + 3]);
+  }
+  __syncthreads();  // bin starts
+#pragma unroll
+  for (uint32_t t = 0; t < S; ++t)
+    if (t * NT + tid < len) srt[hist[bp[t] >> 16] + (bp[t] & 0xFFFFu)] = k[t];
+  __syncthreads();  // keys in bin order
+  lo_out = lo;
+  nbits_out = nbits;
+  for (uint32_t q1 = 0; q1 < q_cnt; q1 += NT) {  // uniform
+    // one rank a thread; the crowded ones are listed (16 bytes each)
+    if (q1 + tid < q_cnt) {
+      const Query q = q1 == 0 ? q0 : cq[q1 + tid];
+      const uint32_t r = q.rank - 1;
+      KT x = srt[r];
+      const uint32_t e = coarse[(uint32_t)(x >> sh)];
+      const uint32_t low = sh == 0 ? 0u : sh <= 32 ? (uint32_t)x << (32 - sh) : (uint32_t)(x >> (sh - 32));
+      const uint32_t bn = (e & 0xFFFFu) + __umulhi(low, e >> 16);
+      const uint32_t s0 = hist[bn], m = (bn + 1 < FB ? hist[bn + 1] : len) - s0;
+      if (sh > 0 && m > kBinThread) {
+        list[atomicAdd(&nlist, 1u)] = make_uint4(s0, m, r - s0, q.out);
+        atomicAdd(&work, m);
+      } else {
+        if (sh > 0 && m > 1) {
+          // the bin's keys in registers (copies of the last key past its
+          // end), each one's rank by comparing every pair once
+          KT y[kBinThread];
+          uint32_t below[kBinThread];
+#pragma unroll
+          for (uint32_t j = 0; j < kBinThread; ++j) {
+            y[j] = srt[s0 + min(j, m - 1)];
+            below[j] = 0;
+          }
+#pragma unroll
+          for (uint32_t j = 1; j < kBinThread; ++j) {
+#pragma unroll
+            for (uint32_t c = 0; c < j; ++c) {
+              const bool lt = j < m && y[j] < y[c];  // the earlier one first on a tie
+              below[c] += lt ? 1u : 0u;
+              below[j] += lt ? 0u : 1u;
+            }
+          }
+#pragma unroll
+          for (uint32_t j = 0; j < kBinThread; ++j) x = j < m && below[j] == r - s0 ? y[j] : x;
+        }
+        out[q.out] = from_key<C>((KT)(lo + x));
+      }
+    }
+    __syncthreads();  // the list is complete
+    const uint32_t nl = nlist;
+    if (work > kBinWork) return false;  // uniform
+    for (uint32_t li = w; li < nl; li += NW) {
+      const uint4 it = list[li];
+      const KT* p = srt + it.x;
+      const uint32_t m = it.y;
+      uint32_t r = it.z;
+      KT x;
+      if (m <= 64) {
+        // a key a lane; ties broken by position (copies of one value: that one)
+        x = p[min(lane, m - 1)];
+        if (__ballot(x != wave_lane<KT>(x, 0)) != 0) {
+          uint32_t below = 0;
+          for (uint32_t j = 0; j < m; ++j) {
+            const KT o = wave_lane<KT>(x, j);
+            below += (o < x || (o == x && j < lane)) ? 1u : 0u;
+          }
+          const int src = __ffsll((unsigned long long)__ballot(lane < m && below == r)) - 1;
+          x = wave_lane<KT>(x, (uint32_t)src);
+        }
+      } else {
+        uint32_t* const bins = whist + w * 256;
+        bool other = false;  // copies of one value need no digits
+        x = p[0];
+        for (uint32_t i = lane; i < m; i += 64) other = other || p[i] != x;
+        if (__ballot(other) != 0) {
+          int rem = sh;
+          KT pre = (KT)(x >> sh);
+          while (rem > 0) {
+            const int d = rem < 8 ? rem : 8, shift = rem - d;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bins[lane * 4 + j] = 0;
+            wave_sync();
+#pragma unroll 4
+            for (uint32_t i = lane; i < m; i += 64) {
+              const KT v = p[i];
+              if ((KT)(v >> rem) == pre) atomicAdd(&bins[(uint32_t)(v >> shift) & ((1u << d) - 1u)], 1u);
+            }
+            wave_sync();
+            uint32_t bn, below;
+            wave_pick256(bins, lane, r, bn, below);
+            r -= below;
+            pre = (KT)((pre << d) | (KT)bn);
+            rem = shift;
+            wave_sync();
+          }
+          x = pre;
+        }
+      }
+      if (lane == 0) out[it.w] = from_key<C>((KT)(lo + x));
+    }
+    __syncthreads();  // the list is read
+    if (tid == 0) {
+      nlist = 0;
+      work = 0;
+    }
+    __syncthreads();
+  }
+  return true;
+}
+
 // Finisher for children with at most kWaveRanks ranks, and for children
 // with many ranks that fit kSortCap keys: one 256-thread work-group per child
 // (several per CU).  The first kind takes two passes over the child's keys
@@ -2461,7 +2716,7 @@ __device__ __forceinline__ void wave_pick256(const uint32_t* h, uint32_t lane, u
 // bucket) into LDS, where wavefront 0 resolves the rank: by counting for up
 // to 64 keys, by 8-bit radix passes over LDS up to the gather capacity, and
 // beyond it (heavy duplicates of one digit) by 8-bit radix passes over the
-// child in memory.  The second kind is sorted in LDS and every rank read off.
+// child in memory.  The second kind goes through bin_select.
 // R is the number of 16-byte words of a child a thread holds in registers.
 template <typename KT, int C, int R, int X>
 __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
@@ -2483,7 +2738,17 @@ __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
   KT* buf = reinterpret_cast<KT*>(h);  // gathered keys (after the histogram is read)
   uint32_t* bins = h + kFCollectWords;  // 256 bins for the LDS radix passes
   __shared__ uint32_t list[kFThreads + 1];  // this window's children for this finisher; count
-  __shared__ uint4 gk_ext[X > 0 ? X * kFThreads : 1];  // the child's keys past the registers
+  // one child's space past h: its keys past the registers, or a child with
+  // many ranks' list (a word a rank), fine and coarse bins, wavefront
+  // histograms
+  constexpr uint32_t SORTW =
+      kFThreads + kFineBins<kFThreads> / 4 + kFThreads / 4 + kFThreads / 64 * 256 / 4;
+  __shared__ uint4 gk_ext[X * kFThreads > SORTW ? X * kFThreads : SORTW];
+  __shared__ uint32_t smisc[kFThreads / 64 + 2];
+  uint4* const slist = gk_ext;
+  uint32_t* const sbins = reinterpret_cast<uint32_t*>(gk_ext + kFThreads);
+  uint32_t* const scoarse = sbins + kFineBins<kFThreads>;
+  uint32_t* const swave = scoarse + kFThreads;
   // this work-group's children are blockIdx.x, + gridDim.x, ...; they are
   // screened kFThreads at a time, one per thread, and only those for this
   // finisher are walked
@@ -2507,19 +2772,27 @@ __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
       const KT* srcp = (c.src == 0 ? input : (c.src == 1 ? red : red2)) + c.start;
       const Query* __restrict__ cq = c.src == 2 ? cq2 : cq0;
       if (sort_child(c)) {  // uniform
-        // many ranks: the converted keys sorted ascending in LDS (bitonic,
-        // one compare-exchange pair per thread step); rank r is the r-th key
+        // many ranks of a short child; where many of its keys share a few
+        // bins, the keys (minus lo) sorted ascending in LDS: rank r is the
+        // r-th key
         KT* keys = reinterpret_cast<KT*>(h);
         const uint32_t len = (uint32_t)c.len;
+        KT lo;
+        int nbits;
+        if (bin_select<KT, C, kFThreads, kSortCap / kFThreads>(srcp, len, cq + c.q_off, c.q_cnt, out,
+                                                               keys, sbins, scoarse, swave, slist,
+                                                               red_lo, red_hi, smisc, lo, nbits)) {
+          __syncthreads();
+          continue;
+        }
         uint32_t np = 1;
         while (np < len) np <<= 1;
-        for (uint32_t i = tid; i < np; i += kFThreads)
-          keys[i] = i < len ? to_key<C>(srcp[i]) : KeyBits<KT>::MAX;
+        for (uint32_t i = len + tid; i < np; i += kFThreads) keys[i] = KeyBits<KT>::MAX;
         __syncthreads();
         lds_bitonic_sort<kFThreads, kSortCap / 2 / kFThreads>(keys, np);
         for (uint32_t i = tid; i < c.q_cnt; i += kFThreads) {
           const Query q = cq[c.q_off + i];
-          out[q.out] = from_key<C>(keys[q.rank - 1]);
+          out[q.out] = from_key<C>((KT)(lo + keys[q.rank - 1]));
         }
         __syncthreads();
         continue;
@@ -2721,7 +2994,11 @@ constexpr uint32_t kFinishOffRed = kFinishOffGpre + (kGroupMax + 2) * 8;
 constexpr uint32_t kFinishOffGfirst = kFinishOffRed + 32 * 8;
 constexpr uint32_t kFinishOffMisc = kFinishOffGfirst + ((kQCap + 1) * 4 + 15) / 16 * 16;
 constexpr uint32_t kFinishOffList = kFinishOffMisc + 32 * 4;
-constexpr uint32_t kFinishLdsTotal = kFinishOffList + (kThreads + 4) * 4;
+constexpr uint32_t kFinishOffWave = (kFinishOffList + (kThreads + 4) * 4 + 15) / 16 * 16;
+constexpr uint32_t kFinishLdsTotal = kFinishOffWave + kThreads / 64 * 256 * 4;
+static_assert(kGroupMax * 256 >= kFineBins<kThreads> && kQCap >= kThreads, "bin_select's bins fit");
+static_assert(kThreads <= kQCap, "bin_select's list fits the query arrays");
+static_assert(kThreads / 64 + 2 <= 32, "bin_select's totals fit the misc words");
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ input,
                                                      const KT* __restrict__ red,
@@ -2749,6 +3026,8 @@ __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ inpu
   uint32_t* misc = reinterpret_cast<uint32_t*>(base + kFinishOffMisc);      // 32 words
   uint32_t* list = reinterpret_cast<uint32_t*>(base + kFinishOffList);      // kThreads + count
   uint32_t& nlist = list[kThreads];
+  uint32_t* whist = reinterpret_cast<uint32_t*>(base + kFinishOffWave);     // 256 a wavefront
+  uint4* blist = reinterpret_cast<uint4*>(qv);                              // qv and qpre
   const uint32_t tid = threadIdx.x;
 
   // this work-group's children are blockIdx.x, + gridDim.x, ...; they are
@@ -2773,65 +3052,52 @@ __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ inpu
       const Query* __restrict__ cq = c.src == 2 ? cq2 : cq0;
       const bool inl = c.len <= CAP;
       KT lo = (KT)c.lo, hi = (KT)c.hi;
-      if (inl) {  // the child into LDS, eight loads per thread in flight
-        constexpr uint32_t D = 8;
-        for (uint32_t i0 = 0; i0 < c.len; i0 += D * kThreads) {
-          KT v[D];
-#pragma unroll
-          for (uint32_t u = 0; u < D; ++u) {
-            const uint32_t i = i0 + u * kThreads + tid;
-            if (i < c.len) v[u] = srcp[i];
+      int nbits;
+      if (inl) {
+        if (bin_select<KT, C, kThreads, CAP / kThreads>(srcp, (uint32_t)c.len, cq + c.q_off, c.q_cnt,
+                                                        out, keys, hist, gfirst, whist, blist,
+                                                        red_lo, red_hi, misc, lo, nbits)) {
+          __syncthreads();
+          continue;
+        }
+        // crowded bins under many ranks; keys holds the child minus lo
+        if (c.q_cnt > kSortRanks || c.len <= kSortLen) {
+          // sort the keys in LDS, then every rank is a lookup
+          const uint32_t np = ((uint32_t)c.len + kThreads - 1) / kThreads * kThreads;
+          for (uint32_t i = c.len + tid; i < np; i += kThreads) keys[i] = KeyBits<KT>::MAX;
+          __syncthreads();
+          lds_radix_sort<KT, CAP / kThreads>(keys, np, nbits, hist, misc);
+          for (uint32_t i = tid; i < c.q_cnt; i += kThreads) {
+            Query q = cq[c.q_off + i];
+            out[q.out] = from_key<C>((KT)(lo + keys[q.rank - 1]));
           }
-#pragma unroll
-          for (uint32_t u = 0; u < D; ++u) {
-            const uint32_t i = i0 + u * kThreads + tid;
-            if (i < c.len) keys[i] = to_key<C>(v[u]);
+          __syncthreads();
+          continue;
+        }
+      } else {
+        if (c.need_range) {
+          KT a = KeyBits<KT>::MAX, b = 0;
+          for_each_elem(srcp, c.len, [&](KT raw) {  // 16-byte loads, four in flight per thread
+            const KT k = to_key<C>(raw);
+            a = k < a ? k : a;
+            b = k > b ? k : b;
+          });
+          for (int d = 32; d >= 1; d >>= 1) {
+            KT x = __shfl_xor(a, d, 64), y = __shfl_xor(b, d, 64);
+            a = x < a ? x : a;
+            b = y > b ? y : b;
+          }
+          if (lane_id() == 0) { red_lo[tid >> 6] = a; red_hi[tid >> 6] = b; }
+          __syncthreads();
+          lo = red_lo[0]; hi = red_hi[0];
+          for (int w = 1; w < 16; ++w) {
+            lo = red_lo[w] < lo ? red_lo[w] : lo;
+            hi = red_hi[w] > hi ? red_hi[w] : hi;
           }
         }
-      }
-      if (c.need_range) {
-        KT a = KeyBits<KT>::MAX, b = 0;
-        auto mm = [&](KT k) {
-          a = k < a ? k : a;
-          b = k > b ? k : b;
-        };
-        if (inl) {
-          for (uint32_t i = tid; i < c.len; i += kThreads) mm(keys[i]);
-        } else {  // 16-byte loads, four in flight per thread
-          for_each_elem(srcp, c.len, [&](KT raw) { mm(to_key<C>(raw)); });
-        }
-        for (int d = 32; d >= 1; d >>= 1) {
-          KT x = __shfl_xor(a, d, 64), y = __shfl_xor(b, d, 64);
-          a = x < a ? x : a;
-          b = y > b ? y : b;
-        }
-        if (lane_id() == 0) { red_lo[tid >> 6] = a; red_hi[tid >> 6] = b; }
-        __syncthreads();
-        lo = red_lo[0]; hi = red_hi[0];
-        for (int w = 1; w < 16; ++w) {
-          lo = red_lo[w] < lo ? red_lo[w] : lo;
-          hi = red_hi[w] > hi ? red_hi[w] : hi;
-        }
+        nbits = bitlen<KT>(hi - lo);
       }
       __syncthreads();
-      if (inl) {
-        for (uint32_t i = tid; i < c.len; i += kThreads) keys[i] -= lo;
-      }
-      const int nbits = bitlen<KT>(hi - lo);
-
-      if (inl && (c.q_cnt > kSortRanks || c.len <= kSortLen)) {
-        // many ranks or a short child: sort its keys in LDS, then every rank is a lookup
-        const uint32_t np = ((uint32_t)c.len + kThreads - 1) / kThreads * kThreads;
-        for (uint32_t i = c.len + tid; i < np; i += kThreads) keys[i] = KeyBits<KT>::MAX;
-        __syncthreads();
-        lds_radix_sort<KT, CAP / kThreads>(keys, np, nbits, hist, misc);
-        for (uint32_t i = tid; i < c.q_cnt; i += kThreads) {
-          Query q = cq[c.q_off + i];
-          out[q.out] = from_key<C>((KT)(lo + keys[q.rank - 1]));
-        }
-        __syncthreads();
-        continue;
-      }
 
       for (uint32_t q0 = 0; q0 < c.q_cnt; q0 += kQCap) {
         const uint32_t nq = min(kQCap, c.q_cnt - q0);

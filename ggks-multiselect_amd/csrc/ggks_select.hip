@@ -277,8 +277,8 @@ static void level_attrs(const Plan&) {
 template <typename KT, int C>
 static void finish(hipStream_t s, const KT* d_src, const KT* red, const KT* red2,
                    const Child* kids, uint32_t n, const Query* cq, const Query* cq2, KT* d_out,
-                   uint32_t max_groups, bool lite, bool big, const uint32_t* bigw) {
-  bool launched = false;
+                   uint32_t max_groups, bool lite, bool small, bool big, const uint32_t* bigw) {
+  bool launched = !small;  // small = false: no child for the 256-thread finisher
   if constexpr (sizeof(KT) == 4) {
     if (lite) {
       hipLaunchKernelGGL((k_finish_small_lite<KT, C>), dim3(std::min<uint32_t>(n, 65536)),
@@ -320,15 +320,15 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
   // an engine segment's by its mean bucket size
   const uint64_t lite_keys = finish_small_reg_keys<KT>(true);
   const bool dlite = p.dmax_keys <= lite_keys, elite = 2 * p.emax_keys <= lite_keys;
-  // whether a direct child (planned on the host) is one for k_finish; a plan
-  // without its host tables (the no-allocation path) may have one
-  bool dbig = ndirect > 0 && p.direct_children.empty();
-  for (const Child& c : p.direct_children) dbig = dbig || big_child(c.len, c.q_cnt);
+  // which finishers the direct children (planned on the host) are for; a plan
+  // without its host tables (the no-allocation path) may have either
+  bool dbig = ndirect > 0 && p.direct_children.empty(), dsmall = dbig;
+  for (const Child& c : p.direct_children) (big_child(c.len, c.q_cnt) ? dbig : dsmall) = true;
   auto finish_direct = [&](hipStream_t ds) {
     const Child* dk = reinterpret_cast<const Child*>(A + p.off_dchildren);
     const Query* dq = reinterpret_cast<const Query*>(A + p.off_dqueries);
     finish<KT, C>(ds, d_src, (const KT*)nullptr, (const KT*)nullptr, dk, ndirect, dq,
-                  (const Query*)nullptr, d_out, 256, dlite, dbig, (const uint32_t*)nullptr);
+                  (const Query*)nullptr, d_out, 256, dlite, dsmall, dbig, (const uint32_t*)nullptr);
   };
   const uint32_t nseg = p.nsegs;
   if (nseg > 0) {
@@ -426,7 +426,7 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
                          l2count, p.cmax, rows2, bits2, wb2, red2);
     }
     // the second level's children are not counted: k_finish screens them
-    finish<KT, C>(s, d_src, red, red2, kids, p.nq, cq, cq2, d_out, 256, elite, true,
+    finish<KT, C>(s, d_src, red, red2, kids, p.nq, cq, cq2, d_out, 256, elite, true, true,
                   p.level2 ? (const uint32_t*)nullptr : bigw);
   } else {
     for (int st = 1; st < GGKS_NSTAGES; ++st) stage(x, st);
