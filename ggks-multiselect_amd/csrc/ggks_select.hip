@@ -255,6 +255,7 @@ template <typename KT, int C>
 static void level_attrs(const Plan&) {
   static const bool once = [] {
     set_lds_limit(k_count<KT, C>, ((size_t)kMaxBuckets + kLaneSlots + (1u << kMaxPrefixBits)) * 4);
+    set_lds_limit(k_count_small<KT, C>, ((size_t)CompactCfg<true>::buckets + kLaneSlots + CompactCfg<true>::lut_words) * 4);
     set_lds_limit(k_findk<KT, C>, ((size_t)kMaxBuckets + (1u << kMaxPrefixBits) +
                                    3 * ((kMaxBuckets + 31) / 32) + 32) * 4);
     set_lds_limit(k_findk_small<KT, C>, ((size_t)kFindkSmallBuckets + (1u << kMaxPrefixBits) +
@@ -382,9 +383,13 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
       finish_direct(x.side);
       HIP_TRY(hipEventRecord(x.join, x.side));
     }
-    launch_stage(x.prof, 3, k_count<KT, C>, dim3(nchunks), dim3(kThreads),
-                 (uint32_t)(((size_t)p.bmax_max + kLaneSlots + (1u << p.pbits_max)) * 4), s, d_src, segs, states,
-                 chunks, lut, rows);
+    const uint32_t clds = (uint32_t)(((size_t)p.bmax_max + kLaneSlots + (1u << p.pbits_max)) * 4);
+    if (compact_small(p.pbits_max, p.bmax_max))
+      launch_stage(x.prof, 3, k_count_small<KT, C>, dim3(nchunks), dim3(kThreads), clds, s, d_src,
+                   segs, states, chunks, lut, rows);
+    else
+      launch_stage(x.prof, 3, k_count<KT, C>, dim3(nchunks), dim3(kThreads), clds, s, d_src, segs,
+                   states, chunks, lut, rows);
     stage(x, 4);
     hipLaunchKernelGGL(k_reduce, dim3(p.nitems), dim3(kThreads), 0, s, segs,
                        states, items, rows, tot, gsum);
