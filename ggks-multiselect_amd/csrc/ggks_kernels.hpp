@@ -95,6 +95,12 @@ __device__ __forceinline__ uint32_t wave_last(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Lane l's value (l uniform).
 template <typename KT>
 __device__ __forceinline__ KT wave_lane(KT v, uint32_t l) {
@@ -736,6 +742,87 @@ constexpr uint64_t finish_small_reg_keys(bool lite) {
 // block's kThreads samples (3.1 %): it then gets a bucket of its own.
 constexpr uint32_t kHeavyMinCount = 32;
 
+// Mark the buckets that can hold a segment's ranks.  A rank r of n has about
+// x = r S / n of the S samples below it, give or take the binomial deviation:
+// its bucket lies between those of sample positions x - d and x + d with
+// d = 3 sqrt(x (1 - x / S)) + 5 (a miss only costs the second pass).  Of a
+// prefix with few samples, all sub-buckets count; so they do where the prefixes
+// beside it hold a third fewer or half more samples (a density that falls or
+// ends inside the prefix puts its keys at one end).  Inside any other prefix,
+// positions are spread evenly, with a sixteenth of it to spare on each side
+// for a slope of that size.  A rank whose span is too wide for the whole to qualify sets *wide.
+__device__ __forceinline__ void predict(const uint32_t* cum, const uint32_t* ent, const uint32_t* cnt,
+                                        uint32_t P, uint32_t B, uint32_t S, const SegDesc& sd,
+                                        uint32_t myk, uint32_t* mark, uint32_t* wide) {
+  const uint32_t tid = threadIdx.x;
+  const float fs = (float)S;
+  // the prefix holding sample position u < S
+  auto prefix_of = [&](uint32_t u) {
+    uint32_t a = 0, z = P - 1;  // smallest p with cum[p] + cnt[p] > u
+    while (a < z) {
+      const uint32_t m = (a + z) >> 1;
+      if (cum[m] + cnt[m] > u) z = m; else a = m + 1;
+    }
+    return a;
+  };
+  auto even = [&](uint32_t p) {
+    const uint32_t c = cnt[p], c0 = p > 0 ? cnt[p - 1] : 0u, c1 = p + 1 < P ? cnt[p + 1] : 0u;
+    return c > S / 64 && 3 * c0 >= 2 * c && 2 * c0 <= 3 * c && 3 * c1 >= 2 * c && 2 * c1 <= 3 * c;
+  };
+  auto span = [&](uint64_t rank, uint32_t& blo, uint32_t& bhi) {
+    const float x = ((float)rank - 0.5f) / (float)sd.len * fs;
+    const float d = 3.f * sqrtf(fmaxf(0.f, x * (1.f - x / fs))) + 5.f;
+    blo = 0;
+    bhi = B - 1;
+    if (x - d > 0.f) {
+      const uint32_t u = min((uint32_t)(x - d), S - 1), p = prefix_of(u), nb = ent[p] >> 16;
+      const uint32_t j = even(p) ? (uint32_t)((uint64_t)nb * (u - cum[p]) / cnt[p]) : 0u, sl = nb / 16 + 1;
+      blo = (ent[p] & 0xFFFFu) + (j > sl ? j - sl : 0u);
+    }
+    if (x + d + 1.f < fs) {
+      const uint32_t u = min((uint32_t)(x + d) + 1u, S - 1), p = prefix_of(u), nb = ent[p] >> 16;
+      const uint32_t j = even(p) ? (uint32_t)((uint64_t)nb * (u - cum[p]) / cnt[p]) + nb / 16 + 1 : nb;
+      bhi = (ent[p] & 0xFFFFu) + min(j, nb - 1);
+    }
+    if ((uint64_t)(bhi - blo) * kSpecShare > B) *wide = 1u;
+  };
+  // the bits of [a, z] (a <= z < B) from word first, step words apart
+  auto mark_range = [&](uint32_t a, uint32_t z, uint32_t first, uint32_t step) {
+    for (uint32_t w = (a >> 5) + first; w <= (z >> 5); w += step) {
+      uint32_t m = ~0u;
+      if (w == (a >> 5)) m &= ~0u << (a & 31u);
+      if (w == (z >> 5)) m &= ~0u >> (31u - (z & 31u));
+      atomicOr(&mark[w], m);
+    }
+  };
+  if (sd.qsrc == QSRC_TOPK) {  // every rank from len - K + 1 up
+    uint32_t blo, bhi;
+    span(sd.len - sd.q_cnt + 1, blo, bhi);
+    if ((uint64_t)(B - 1 - blo) * kSpecShare > B) {
+      if (tid == 0) *wide = 1u;
+      return;
+    }
+    mark_range(blo, B - 1, tid, kThreads);
+    return;
+  }
+  // one rank a thread; a k list is mostly sorted, so a lane marks only what
+  // the lane before it does not
+  const bool ok = tid < sd.q_cnt;
+  uint32_t blo = 1, bhi = 0;
+  if (ok) {
+    const uint32_t k = myk < 1 || (uint64_t)myk > sd.len ? 1u : myk;
+    span(sd.len - k + 1, blo, bhi);
+  }
+  const uint32_t plo = (uint32_t)__shfl_up((int)blo, 1, 64), phi = (uint32_t)__shfl_up((int)bhi, 1, 64);
+  if (!ok || (uint64_t)(bhi - blo) * kSpecShare > B) return;  // no shuffles below
+  if (lane_id() == 0 || plo > bhi || phi < blo || (uint64_t)(phi - plo) * kSpecShare > B) {
+    mark_range(blo, bhi, 0, 1);
+    return;
+  }
+  if (blo < plo) mark_range(blo, plo - 1, 0, 1);
+  if (bhi > phi) mark_range(phi + 1, bhi, 0, 1);
+}
+
 // Build one segment's bucket function (one block per segment).
 //  MODE_SAMPLE  prefixes of 2^s keys over the sampled range, sub-buckets in
 //               proportion to each prefix's share of the sample; a run of
@@ -756,7 +843,9 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
                                                   uint32_t* __restrict__ lut_pool,
                                                   uint32_t* __restrict__ l2count,
                                                   uint32_t* __restrict__ bigw,
-                                                  uint32_t* __restrict__ hgram) {
+                                                  uint32_t* __restrict__ hgram,
+                                                  const uint32_t* __restrict__ kraw,
+                                                  uint32_t* __restrict__ bits_pool) {
   // the second level's counters (heavy children, chunks) start at zero in
   // every run; k_findk, which counts them, runs after this kernel
   if (l2count && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2) l2count[threadIdx.x] = 0;
@@ -772,10 +861,13 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   __shared__ uint32_t wsum[17];
   __shared__ KT red_lo[16], red_hi[16];
   __shared__ KT sh_hv;
-  __shared__ uint32_t sh_hvon, sh_last;
+  __shared__ uint32_t sh_hvon, sh_last, sh_wide, sh_cand, sh_cells[2];
   constexpr uint32_t W = KeyBits<KT>::W;
   const SegDesc sd = segs[blockIdx.x];
   const uint32_t tid = threadIdx.x;
+  // ranks to predict: this thread's k, read now so that it arrives early
+  const bool spec_k = (sd.flags & SEG_SPEC) && sd.qsrc == QSRC_K;  // at most kSpecRanks
+  const uint32_t myk = spec_k && tid < sd.q_cnt ? kraw[sd.q_off + tid] : 0u;
   // k_sample's prefix counts, loaded now (16 bytes a thread) so that they
   // arrive while the sample's range is reduced; used for full-width ranges
   const bool hload = hgram && sd.mode == MODE_SAMPLE && tid < (1u << sd.pbits) / 4;
@@ -785,6 +877,7 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   const uint32_t nparts = min(lut_parts(sd.mode, sd.nsample, sizeof(KT)), gridDim.y), part = blockIdx.y;
   if (part >= nparts) return;  // uniform
   uint32_t* lut = lut_pool + sd.lut_off;
+  if (tid < 2) sh_cells[tid] = 0;
   KT kmin, kmax;
   uint32_t pb = sd.pbits;
   uint32_t hvon = 0;
@@ -825,6 +918,10 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
     }
     hvon = sh_hvon;
     hv = sh_hv;
+    if (spec_k && tid < sd.q_cnt) {
+      const uint32_t cell = (uint32_t)min((uint64_t)myk * 64 / sd.len, (uint64_t)63);
+      atomicOr(&sh_cells[cell >> 5], 1u << (cell & 31u));
+    }
   } else {
     kmin = (KT)sd.lo;
     kmax = (KT)sd.hi;
@@ -877,7 +974,8 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   }
   const uint32_t Bt = sd.bmax - (hvon ? 2u : 0u);  // bucket budget of L
   const uint32_t cap = s >= 16 ? 65535u : min(65535u, 1u << s);
-  uint32_t Btot;
+  uint32_t Btot, nsum = 0;
+  bool spec = false;
 
   if (sd.mode == MODE_RADIX) {
     for (uint32_t p = tid; p < P; p += kThreads) {
@@ -968,15 +1066,45 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
     for (uint32_t p = p0; p < p1; ++p) local += width(p, nbv);
     uint32_t tot;
     uint32_t run = block_excl_scan(local, wsum, tot);
+    // (ranks in many of 64 even cells of the vector never fit in the share:
+    // sh_cells holds the cells taken, behind the barriers above)
+    spec = (sd.flags & SEG_SPEC) && sd.qsrc != QSRC_QUERIES && !hvon && t3 > 0 &&
+           __popc(sh_cells[0]) + __popc(sh_cells[1]) <= kSpecCells;  // uniform
+    nsum = t3;
+    uint32_t crun = 0;
+    if (__builtin_expect(spec, 0)) {
+      uint32_t c = 0, call;
+      for (uint32_t p = p0; p < p1; ++p) c += cnt[p];
+      crun = block_excl_scan(c, wsum, call);
+    }
     for (uint32_t p = p0; p < p1; ++p) {
       const uint32_t w = width(p, nbv);
       const uint32_t base = (w == 0) ? run - 1 : run;  // a run's later prefixes
       lut[p] = base | (nbv << 16);
+      if (spec) {  // samples below the prefix, and its entry (cnt4 is free now)
+        cnt4[p] = crun;
+        cnt4[(1u << kMaxPrefixBits) + p] = base | (nbv << 16);
+        crun += cnt[p];
+      }
       run += w;
     }
     Btot = tot;
   }
+  uint32_t* const mark = cnt4 + (2u << kMaxPrefixBits);  // candidate buckets, a bit each
+  const uint32_t nmark = (Btot + 31) / 32;
+  if (__builtin_expect(spec, 0)) {
+    for (uint32_t i = tid; i < nmark; i += kThreads) mark[i] = 0;
+    if (tid == 0) sh_wide = sh_cand = 0;
+  }
   __syncthreads();  // the LUT is complete (thread 0 reads hv's entry)
+  if (__builtin_expect(spec, 0)) {
+    predict(cnt4, cnt4 + (1u << kMaxPrefixBits), cnt, P, Btot, nsum, sd, myk, mark, &sh_wide);
+    __syncthreads();
+    if (tid < nmark && mark[tid]) atomicAdd(&sh_cand, (uint32_t)__popc(mark[tid]));
+    __syncthreads();
+    spec = !sh_wide && sh_cand * kSpecShare <= Btot;
+    if (spec && tid < nmark) bits_pool[sd.bits_off + tid] = mark[tid];
+  }
   if (tid == 0) {
     SegState st = {};
     st.kb = (uint64_t)kb;
@@ -997,6 +1125,7 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
     st.hvon = 0;
     st.hv = 0;
     st.hb = 0;
+    st.arrive = spec ? 1u : 0u;
     if (hvon) {  // hv's bucket is L(hv) + 1; two more buckets in all
       BucketFn<KT> fn;
       fn.init(st);
@@ -1015,13 +1144,20 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
 
 // Pass 1: per-chunk LDS histogram of bucket ids.
 constexpr uint32_t kLaneSlots = 64;  // k_count's per-lane heavy-bin slots
+// A wavefront's stage of candidates: what is left of the LDS beside 2^15
+// buckets and 2^12 prefixes.
+constexpr uint32_t kStageBytes = 992;
+static_assert((kMaxBuckets + kLaneSlots + (1u << kMaxPrefixBits)) * 4 + kThreads / 64 * kStageBytes + 8 <=
+                  160 * 1024, "LDS of the count pass");
 template <typename KT, int C, int R>
 __device__ __forceinline__ void count_chunk(const KT* __restrict__ src,
                                             const SegDesc* __restrict__ segs,
                                             const SegState* __restrict__ states,
                                             const Chunk* __restrict__ chunks,
                                             const uint32_t* __restrict__ lut_pool,
-                                            uint32_t* __restrict__ rows) {
+                                            uint32_t* __restrict__ rows,
+                                            const uint32_t* __restrict__ bits_pool,
+                                            KT* __restrict__ red, KT* __restrict__ samples) {
   extern __shared__ uint32_t lds[];
   const Chunk ch = chunks[blockIdx.x];
   const SegDesc& sd = segs[ch.seg];
@@ -1052,14 +1188,52 @@ __device__ __forceinline__ void count_chunk(const KT* __restrict__ src,
 #pragma unroll
     for (int t = 0; t < R; ++t) v[t] = stream_load(&pv[(uint64_t)t * kThreads + tid]);
   }
-  for (uint32_t i = threadIdx.x; i < st.B; i += kThreads) hist[i] = 0;
+  // candidates (kSpecShare): a candidate bucket's bin has its top bit set from
+  // the start, so the count's own atomic, asked for the old value, tells
+  // which keys to keep: no further look-up and no table of buckets
+  // Each wavefront gathers them in a stage of its own and stores a stageful at
+  // a time (no barrier; a store every round made the wait for the next
+  // round's loads one for the stores too: 2^27 floats with 2 % candidates
+  // counted in 112 us, 103 staged, 88 without candidates).
+  const bool spec = st.arrive != 0;  // uniform
+  __shared__ uint32_t ncand;
+  constexpr uint32_t STAGE = kStageBytes / sizeof(KT);
+  __shared__ KT stage[kThreads / 64][STAGE];
+  uint32_t nst = 0;  // keys in this wavefront's stage (uniform)
+  KT* const area = red + sd.red_base + spec_area(sd.len, ch.start);
+  const uint32_t acap = (uint32_t)(len >> kSpecAreaLog2);
+  if (__builtin_expect(spec, 0)) {  // (kept out of the others' straight line)
+    const uint32_t* bm = bits_pool + sd.bits_off;
+    for (uint32_t i = threadIdx.x; i < st.B; i += kThreads) hist[i] = (bm[i >> 5] >> (i & 31u)) << 31;
+    if (threadIdx.x == 0) ncand = 0;
+  } else {
+    for (uint32_t i = threadIdx.x; i < st.B; i += kThreads) hist[i] = 0;
+  }
   if (threadIdx.x < kLaneSlots) hist[bmax + threadIdx.x] = 0;
   for (uint32_t i = threadIdx.x; i < st.P; i += kThreads) lut[i] = lut_pool[sd.lut_off + i];
   __syncthreads();
   BucketFn<KT> bk;
   bk.init(st);
-  if (tid < head) atomicAdd(&hist[bk(to_key<C>(p[tid]), lut)], 1u);
-  if (done + tid < len) atomicAdd(&hist[bk(to_key<C>(p[done + tid]), lut)], 1u);
+  auto drain = [&]() {
+    uint32_t at = 0;
+    if (lane_id() == 0) at = atomicAdd(&ncand, nst);
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    wave_sync();
+    if (at + nst <= acap)  // uniform (a chunk past its part is read again)
+      for (uint32_t i = lane_id(); i < nst; i += 64) area[at + i] = stage[tid >> 6][i];
+    wave_sync();
+    nst = 0;
+  };
+  auto count_one = [&](KT raw, uint32_t b) {
+    if (__builtin_expect(!spec, 1)) {  // uniform
+      atomicAdd(&hist[b], 1u);
+    } else if (atomicAdd(&hist[b], 1u) >> 31) {
+      const uint32_t at = atomicAdd(&ncand, 1u);
+      if (at < acap) area[at] = raw;
+    }
+  };
+  if (tid < head) count_one(p[tid], bk(to_key<C>(p[tid]), lut));
+  if (done + tid < len) count_one(p[done + tid], bk(to_key<C>(p[done + tid]), lut));
   // full rounds, software pipelined: the next round's loads are in flight
   // while a round is bucketed and counted
   // With a heavy value its bucket takes up to most keys: each lane counts
@@ -1067,7 +1241,7 @@ __device__ __forceinline__ void count_chunk(const KT* __restrict__ src,
   // atomic on one address, no change of the execution mask), and the slots
   // are added into the bucket at the end.
   const uint32_t hbk = st.hb;
-  auto full_rounds = [&](auto left, auto hvt) {
+  auto full_rounds = [&](auto left, auto hvt, auto spc) {
     if (r0 + per_round > nvec) return;  // uniform (round 0's loads are in v)
     for (; r0 + per_round <= nvec; r0 += per_round) {
       KT k[N];
@@ -1082,19 +1256,61 @@ __device__ __forceinline__ void count_chunk(const KT* __restrict__ src,
       if (decltype(hvt)::value) {
 #pragma unroll
         for (int i = 0; i < N; ++i) atomicAdd(&hist[b[i] == hbk ? hslot : b[i]], 1u);
+      } else if (decltype(spc)::value) {
+        uint32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) b[i] = atomicAdd(&hist[b[i]], 1u);
+#pragma unroll
+        for (int i = 0; i < N; ++i) any |= b[i];
+        if (__ballot((int32_t)any < 0)) {  // uniform
+          uint64_t m[N];  // the lanes with a candidate at i (scalar registers)
+          uint32_t tot = 0;
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            m[i] = __ballot((int32_t)b[i] < 0);
+            tot += (uint32_t)__popcll(m[i]);
+          }
+          if (nst + tot > STAGE) drain();  // uniform
+          // (two copies of the stores, to LDS and to memory, so that neither
+          // goes through a generic address, which would wait for both)
+          auto put = [&](KT* dst) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+              if (m[i]) {  // uniform
+                const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(m[i] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[i], 0u));
+                if ((int32_t)b[i] < 0) dst[below] = k[i];
+                dst += __popcll(m[i]);
+              }
+            }
+          };
+          if (tot <= STAGE) {  // uniform
+            put(&stage[tid >> 6][nst]);
+            nst += tot;
+          } else {  // more than the stage holds go straight out
+            uint32_t at = 0;
+            if (lane_id() == 0) at = atomicAdd(&ncand, tot);
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+            if (at + tot <= acap) put(area + at);  // uniform
+          }
+        }
       } else {
 #pragma unroll
         for (int i = 0; i < N; ++i) atomicAdd(&hist[b[i]], 1u);
       }
     }
   };
-  // uniform: the sub-field shift direction and the heavy-value term
-  if (!st.hvon) {
-    if (st.s <= 24) full_rounds(std::true_type{}, std::false_type{});
-    else full_rounds(std::false_type{}, std::false_type{});
+  // uniform: the sub-field shift direction, the heavy-value term, candidates
+  // (none with a heavy value)
+  if (__builtin_expect(spec, 0)) {
+    if (st.s <= 24) full_rounds(std::true_type{}, std::false_type{}, std::true_type{});
+    else full_rounds(std::false_type{}, std::false_type{}, std::true_type{});
+  } else if (!st.hvon) {
+    if (st.s <= 24) full_rounds(std::true_type{}, std::false_type{}, std::false_type{});
+    else full_rounds(std::false_type{}, std::false_type{}, std::false_type{});
   } else {
-    if (st.s <= 24) full_rounds(std::true_type{}, std::true_type{});
-    else full_rounds(std::false_type{}, std::true_type{});
+    if (st.s <= 24) full_rounds(std::true_type{}, std::true_type{}, std::false_type{});
+    else full_rounds(std::false_type{}, std::true_type{}, std::false_type{});
   }
   for (uint64_t i = r0 + tid; i < nvec; i += kThreads) {  // last partial round
     uint4 v[1] = {stream_load(&pv[i])};
@@ -1103,8 +1319,9 @@ __device__ __forceinline__ void count_chunk(const KT* __restrict__ src,
     uint32_t b[VEC];
     bucket_batch<KT, C, VEC>(bk, lut, k, b);
 #pragma unroll
-    for (uint32_t j = 0; j < VEC; ++j) atomicAdd(&hist[b[j]], 1u);
+    for (uint32_t j = 0; j < VEC; ++j) count_one(k[j], b[j]);
   }
+  if (__builtin_expect(nst != 0, 0)) drain();  // uniform
   if (st.hvon) {  // uniform
     __syncthreads();
     if (threadIdx.x < kLaneSlots) {
@@ -1115,16 +1332,24 @@ __device__ __forceinline__ void count_chunk(const KT* __restrict__ src,
   }
   __syncthreads();
   uint32_t* row = rows + sd.row_base + (uint64_t)ch.idx * bmax;
+  if (__builtin_expect(spec, 0)) {  // uniform
+    for (uint32_t i = threadIdx.x; i < st.B; i += kThreads) row[i] = hist[i] & 0x7FFFFFFFu;
+    // the sample is dead; its place (at least 1024 keys, at most 512 chunks)
+    // takes the chunks' candidate counts
+    if (threadIdx.x == 0) reinterpret_cast<uint32_t*>(samples + sd.sample_off)[ch.idx] = ncand;
+    return;
+  }
   for (uint32_t i = threadIdx.x; i < st.B; i += kThreads) row[i] = hist[i];
 }
 
 #define GGKS_COUNT_PARAMS                                                                      \
   const KT *__restrict__ src, const SegDesc *__restrict__ segs,                                \
       const SegState *__restrict__ states, const Chunk *__restrict__ chunks,                   \
-      const uint32_t *__restrict__ lut_pool, uint32_t *__restrict__ rows
+      const uint32_t *__restrict__ lut_pool, uint32_t *__restrict__ rows,                      \
+      const uint32_t *__restrict__ bits_pool, KT *__restrict__ red, KT *__restrict__ samples
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) void k_count(GGKS_COUNT_PARAMS) {
-  count_chunk<KT, C, 4>(src, segs, states, chunks, lut_pool, rows);
+  count_chunk<KT, C, 4>(src, segs, states, chunks, lut_pool, rows, bits_pool, red, samples);
 }
 // Plans of at most 4096 buckets (16 KB of bins; compact_small): two loads a
 // round in at most 64 VGPRs, so that two work-groups share a CU and one
@@ -1134,7 +1359,7 @@ __global__ __launch_bounds__(kThreads) void k_count(GGKS_COUNT_PARAMS) {
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_count_small(
     GGKS_COUNT_PARAMS) {
-  count_chunk<KT, C, 2>(src, segs, states, chunks, lut_pool, rows);
+  count_chunk<KT, C, 2>(src, segs, states, chunks, lut_pool, rows, bits_pool, red, samples);
 }
 #undef GGKS_COUNT_PARAMS
 
@@ -1289,6 +1514,9 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
   uint4 gv = make_uint4(0, 0, 0, 0), lv = make_uint4(0, 0, 0, 0);
   if (tid < ng4) gv = reinterpret_cast<const uint4*>(gsums + sd.tot_off / kReduceBins)[tid];
   if (tid < nl4) lv = reinterpret_cast<const uint4*>(lut_pool + sd.lut_off)[tid];
+  // a candidate word of k_lut's (kSpecShare), where it left any
+  const uint32_t cw =
+      (sd.flags & SEG_SPEC) && tid < wcap ? bits_pool[sd.bits_off + tid] : 0u;
   __shared__ SegState st;
   if (threadIdx.x == 0) st = states[blockIdx.x];
   if (tid < ng4) reinterpret_cast<uint4*>(wc)[tid] = gv;
@@ -1346,14 +1574,18 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
   __syncthreads();
 
   // B: per bitmap word its first child and first reduced slot; the child map
+  // (and, from bit 20 up of the children's scan, the words with an active
+  // bucket that is no candidate of k_lut's)
   uint32_t pc = 0, csum = 0, m = 0;
   if (tid < nwords) {
     m = bits[tid];
-    pc = __popc(m);
+    pc = __popc(m) | (m & ~cw ? 1u << 20 : 0u);
     for (uint32_t mm = m; mm; mm &= mm - 1) csum += count_of(tid * 32 + __ffs(mm) - 1);
   }
   uint32_t U, mtot;
-  const uint32_t ubase = block_excl_scan(pc, wsum, U);
+  const uint32_t ubase = block_excl_scan(pc, wsum, U) & 0xFFFFFu;
+  const bool miss = (U >> 20) != 0;
+  U &= 0xFFFFFu;
   const uint32_t cbase = block_excl_scan(csum, wsum, mtot);
   if (tid < nwords) {
     wb[tid] = ubase;
@@ -1521,6 +1753,9 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
   if (tid == 0) {
     states[blockIdx.x].nact = U;
     states[blockIdx.x].nred = mtot;
+    // the compaction reads the candidates: all there, and its children end
+    // below them
+    states[blockIdx.x].arrive = st.arrive && !miss && mtot <= spec_area(sd.len, 0) ? 1u : 0u;
     if (bigw && lbig) atomicAdd(bigw, lbig);
   }
 }
@@ -1606,7 +1841,8 @@ __device__ __forceinline__ void compact_chunk(const KT* __restrict__ src,
                                               const uint32_t* __restrict__ bits_pool,
                                               const uint32_t* __restrict__ wbase_pool,
                                               const uint2* __restrict__ cinfo,
-                                              KT* __restrict__ red) {
+                                              KT* __restrict__ red,
+                                              const KT* __restrict__ samples) {
   using Cfg = CompactCfg<SMALL>;
   constexpr int kRound = Cfg::round;
   extern __shared__ __align__(16) uint32_t lds[];
@@ -1640,7 +1876,15 @@ __device__ __forceinline__ void compact_chunk(const KT* __restrict__ src,
   KT* kb = reinterpret_cast<KT*>(cur + CURS);
   const uint32_t tid = threadIdx.x, lane = lane_id();
   const KT* p = src + sd.data_off + ch.start;
-  const uint64_t len = ch.len;
+  uint64_t len = ch.len;
+  if (__builtin_expect(st.arrive != 0, 0)) {  // uniform: the chunk's candidates, if its part took them all
+    const uint32_t nc = reinterpret_cast<const uint32_t*>(samples + sd.sample_off)[ch.idx];
+    if (nc <= (len >> kSpecAreaLog2)) {
+      if (nc == 0) return;
+      p = red + sd.red_base + spec_area(sd.len, ch.start);
+      len = nc;
+    }
+  }
   uint64_t mis = ((uintptr_t)p & 15u) / sizeof(KT);
   uint64_t head = mis ? (VEC - mis) : 0;
   if (head > len) head = len;
@@ -2080,25 +2324,25 @@ __device__ __forceinline__ void compact_chunk(const KT* __restrict__ src,
       const SegState *__restrict__ states, const Chunk *__restrict__ chunks,                  \
       const uint32_t *__restrict__ lut_pool, uint32_t *__restrict__ rows,                     \
       const uint32_t *__restrict__ bits_pool, const uint32_t *__restrict__ wbase_pool,        \
-      const uint2 *__restrict__ cinfo, KT *__restrict__ red
+      const uint2 *__restrict__ cinfo, KT *__restrict__ red, const KT *__restrict__ samples
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) void k_compact(GGKS_COMPACT_PARAMS) {
   compact_chunk<KT, C, false, false>(src, segs, states, chunks, lut_pool, rows, bits_pool,
-                                     wbase_pool, cinfo, red);
+                                     wbase_pool, cinfo, red, samples);
 }
 // with cursor windows: for plans with a segment of more ranks than LDS
 // cursors (a separate instance, so the window loop costs the others nothing)
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) void k_compact_win(GGKS_COMPACT_PARAMS) {
   compact_chunk<KT, C, false, true>(src, segs, states, chunks, lut_pool, rows, bits_pool,
-                                    wbase_pool, cinfo, red);
+                                    wbase_pool, cinfo, red, samples);
 }
 // at most 64 VGPRs: two 1024-thread work-groups per CU
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_compact_small(
     GGKS_COMPACT_PARAMS) {
   compact_chunk<KT, C, true, false>(src, segs, states, chunks, lut_pool, rows, bits_pool,
-                                    wbase_pool, cinfo, red);
+                                    wbase_pool, cinfo, red, samples);
 }
 #undef GGKS_COMPACT_PARAMS
 
@@ -2460,12 +2704,6 @@ struct GroupKeys {
   }
 };
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Rank r (0-based) among 256 LDS bins h[0, 2^d) counted by a wavefront: the
 // bin holding it and the number of values in lower bins.
 __device__ __forceinline__ void wave_pick256(const uint32_t* h, uint32_t lane, uint32_t r,
@@ -2518,7 +2756,11 @@ __device__ bool bin_select(const KT* __restrict__ srcp, uint32_t len, const Quer
   constexpr uint32_t NW = NT / 64, FB = kFineBins<NT>, WPT = FB / NT;  // fine bins per thread
   constexpr int BB = NT == 1024 ? 10 : 8;                              // log2 coarse bins
   static_assert(NT == (1u << BB) && WPT % 4 == 0 && S * NT <= 32768, "bins");
-  const uint32_t tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+  // (the thread's index behind an empty asm, so that addresses made from it
+  // are not kept in registers through the caller's other loops)
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const uint32_t lane = tid & 63u, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   // misc: NW wavefront totals, then the list's length and its keys
   uint32_t* const wtot = misc;
   uint32_t& nlist = misc[NW];
@@ -2757,7 +2999,10 @@ __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
   const bool w0 = tid < 64;
   KT* buf = reinterpret_cast<KT*>(h);  // gathered keys (after the histogram is read)
   uint32_t* bins = h + kFCollectWords;  // 256 bins for the LDS radix passes
-  __shared__ uint32_t list[kFThreads + 1];  // this window's children for this finisher; count
+  // this window's children for this finisher, those with few ranks from the
+  // front and those with many from the back (two loops: as branches of one,
+  // either's registers crowded the other's into scratch memory), and counts
+  __shared__ uint32_t list[kFThreads + 2];
   // one child's space past h: its keys past the registers, or a child with
   // many ranks' list (a word a rank), fine and coarse bins, wavefront
   // histograms
@@ -2775,48 +3020,24 @@ __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
   const uint32_t ncand =
       nchildren > blockIdx.x ? (nchildren - blockIdx.x + gridDim.x - 1) / gridDim.x : 0u;
   for (uint32_t wstart = 0; wstart < ncand; wstart += kFThreads) {  // uniform
-    if (tid == 0) list[kFThreads] = 0;
+    if (tid < 2) list[kFThreads + tid] = 0;
     __syncthreads();
     if (wstart + tid < ncand) {
       const uint32_t ci = blockIdx.x + (wstart + tid) * gridDim.x;
       const Child cc = children[ci];
-      if (cc.q_cnt != 0 && (wave_child(cc) || sort_child(cc)))
-        list[atomicAdd(&list[kFThreads], 1u)] = ci;
+      if (cc.q_cnt != 0) {
+        if (wave_child(cc)) list[atomicAdd(&list[kFThreads], 1u)] = ci;
+        else if (sort_child(cc)) list[kFThreads - 1 - atomicAdd(&list[kFThreads + 1], 1u)] = ci;
+      }
     }
     __syncthreads();
-    const uint32_t nl = list[kFThreads];
+    const uint32_t nl = list[kFThreads], ns = list[kFThreads + 1];
     for (uint32_t li = 0; li < nl; ++li) {
       const Child c = children[list[li]];
       // source: the input, the first or the second reduced buffer; a
       // second-level child's ranks are in cq2
       const KT* srcp = (c.src == 0 ? input : (c.src == 1 ? red : red2)) + c.start;
       const Query* __restrict__ cq = c.src == 2 ? cq2 : cq0;
-      if (sort_child(c)) {  // uniform
-        // many ranks of a short child; where many of its keys share a few
-        // bins, the keys (minus lo) sorted ascending in LDS: rank r is the
-        // r-th key
-        KT* keys = reinterpret_cast<KT*>(h);
-        const uint32_t len = (uint32_t)c.len;
-        KT lo;
-        int nbits;
-        if (bin_select<KT, C, kFThreads, kSortCap / kFThreads>(srcp, len, cq + c.q_off, c.q_cnt, out,
-                                                               keys, sbins, scoarse, swave, slist,
-                                                               red_lo, red_hi, smisc, lo, nbits)) {
-          __syncthreads();
-          continue;
-        }
-        uint32_t np = 1;
-        while (np < len) np <<= 1;
-        for (uint32_t i = len + tid; i < np; i += kFThreads) keys[i] = KeyBits<KT>::MAX;
-        __syncthreads();
-        lds_bitonic_sort<kFThreads, kSortCap / 2 / kFThreads>(keys, np);
-        for (uint32_t i = tid; i < c.q_cnt; i += kFThreads) {
-          const Query q = cq[c.q_off + i];
-          out[q.out] = from_key<C>((KT)(lo + keys[q.rank - 1]));
-        }
-        __syncthreads();
-        continue;
-      }
       // the passes over the child's keys, given a visitor of its keys
       auto body = [&](auto&& each) {
         KT lo = (KT)c.lo, hi = (KT)c.hi;
@@ -2979,6 +3200,32 @@ __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
         body([&](auto&& f) { gk.for_each(f); });
       } else {
         body([&](auto&& f) { group_for_each(srcp, c.len, f); });
+      }
+      __syncthreads();
+    }
+    for (uint32_t li = 0; li < ns; ++li) {
+      // many ranks of a short child; where many of its keys share a few
+      // bins, the keys (minus lo) sorted ascending in LDS: rank r is the
+      // r-th key
+      const Child c = children[list[kFThreads - 1 - li]];
+      const KT* srcp = (c.src == 0 ? input : (c.src == 1 ? red : red2)) + c.start;
+      const Query* __restrict__ cq = (c.src == 2 ? cq2 : cq0) + c.q_off;
+      KT* keys = reinterpret_cast<KT*>(h);
+      const uint32_t len = (uint32_t)c.len;
+      KT lo;
+      int nbits;
+      if (!bin_select<KT, C, kFThreads, kSortCap / kFThreads>(srcp, len, cq, c.q_cnt, out, keys, sbins,
+                                                              scoarse, swave, slist, red_lo, red_hi,
+                                                              smisc, lo, nbits)) {
+        uint32_t np = 1;
+        while (np < len) np <<= 1;
+        for (uint32_t i = len + tid; i < np; i += kFThreads) keys[i] = KeyBits<KT>::MAX;
+        __syncthreads();
+        lds_bitonic_sort<kFThreads, kSortCap / 2 / kFThreads>(keys, np);
+        for (uint32_t i = tid; i < c.q_cnt; i += kFThreads) {
+          const Query q = cq[i];
+          out[q.out] = from_key<C>((KT)(lo + keys[q.rank - 1]));
+        }
       }
       __syncthreads();
     }

@@ -133,6 +133,14 @@ inline uint64_t seg_heavy_max(uint64_t len, uint32_t nq) {
   return std::min<uint64_t>(nq, len / (kHeavyKeys + 1));
 }
 
+// Whether a segment's active buckets are worth predicting: a sampled segment
+// whose ranks can lie in few places, long enough for the second pass over it
+// to cost more than the prediction, with chunks whose counts leave a histogram
+// word's top bit free.
+inline bool seg_spec(uint32_t mode, bool topk, uint64_t len, uint64_t chunk, uint32_t nq) {
+  return mode == MODE_SAMPLE && (topk || nq <= kSpecRanks) && len >= kSpecMinLen && chunk <= (1ull << 30);
+}
+
 // Second-level regions at the end of an arena layout (tables and scratch
 // sized by the capacity: hmax heavy children, cmax chunks of kChunk2 keys,
 // red elements in the second reduced buffer, nq query slots).
@@ -222,7 +230,7 @@ inline SegDesc single_segment(const SingleShape& sh, int kind, uint64_t n, uint3
   s.radix_bits = sh.rb;
   s.qsrc = kind == GGKS_KIND_TOPK ? QSRC_TOPK : QSRC_K;
   s.out_off = 0;
-  s.flags = 0;
+  s.flags = seg_spec(sh.mode, kind == GGKS_KIND_TOPK, n, sh.csz, nq) ? SEG_SPEC : 0u;
   return s;
 }
 
@@ -493,7 +501,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     s.radix_bits = rb;
     s.qsrc = topk ? QSRC_TOPK : QSRC_K;
     s.out_off = (uint32_t)g.out_offset;
-    s.flags = 0;
+    s.flags = seg_spec(mode, topk, n, csz, g.num_k) ? SEG_SPEC : 0u;
     if (seg_level2(o, mode)) {
       const uint64_t hm = seg_heavy_max(n, g.num_k);
       if (hm > 0) {

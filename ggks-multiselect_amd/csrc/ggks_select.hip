@@ -375,7 +375,7 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
     uint2* cinfo = reinterpret_cast<uint2*>(A + p.off_cinfo);
     hipLaunchKernelGGL((k_lut<KT>), dim3(nseg, p.lut_parts), dim3(kThreads), 0, s, segs, samples,
                        minmax, states,
-                       lut, l2count, bigw, hg);
+                       lut, l2count, bigw, hg, d_k, bits);
     stage(x, 3);
     if (beside) {  // nseg > 0
       HIP_TRY(hipEventRecord(x.fork, s));
@@ -386,10 +386,10 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
     const uint32_t clds = (uint32_t)(((size_t)p.bmax_max + kLaneSlots + (1u << p.pbits_max)) * 4);
     if (compact_small(p.pbits_max, p.bmax_max))
       launch_stage(x.prof, 3, k_count_small<KT, C>, dim3(nchunks), dim3(kThreads), clds, s, d_src,
-                   segs, states, chunks, lut, rows);
+                   segs, states, chunks, lut, rows, bits, red, samples);
     else
       launch_stage(x.prof, 3, k_count<KT, C>, dim3(nchunks), dim3(kThreads), clds, s, d_src, segs,
-                   states, chunks, lut, rows);
+                   states, chunks, lut, rows, bits, red, samples);
     stage(x, 4);
     hipLaunchKernelGGL(k_reduce, dim3(p.nitems), dim3(kThreads), 0, s, segs,
                        states, items, rows, tot, gsum);
@@ -410,15 +410,15 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
     if (compact_small(p.pbits_max, p.bmax_max))
       launch_stage(x.prof, 6, k_compact_small<KT, C>, dim3(nchunks), dim3(kThreads),
                    (uint32_t)compact_lds_bytes<true>(), s, d_src, segs, states, chunks, lut, rows,
-                   bits, wbase, cinfo, red);
+                   bits, wbase, cinfo, red, samples);
     else if (p.qmax > CompactCfg<false>::template cursors<KT>)  // cursor windows possible
       launch_stage(x.prof, 6, k_compact_win<KT, C>, dim3(nchunks), dim3(kThreads),
                    (uint32_t)compact_lds_bytes<false>(), s, d_src, segs, states, chunks, lut, rows,
-                   bits, wbase, cinfo, red);
+                   bits, wbase, cinfo, red, samples);
     else
       launch_stage(x.prof, 6, k_compact<KT, C>, dim3(nchunks), dim3(kThreads),
                    (uint32_t)compact_lds_bytes<false>(), s, d_src, segs, states, chunks, lut, rows,
-                   bits, wbase, cinfo, red);
+                   bits, wbase, cinfo, red, samples);
     stage(x, 7);
     if (p.level2) {  // the heavy children's second level (part of the finish stage)
       const uint32_t g2 = std::max<uint32_t>(1, std::min<uint32_t>(p.cmax, kLevel2Groups));

@@ -65,7 +65,42 @@ struct SegDesc {          // planned on the host, read-only on the device
   uint32_t flags;         // SEG_LEVEL2: its heavy children go to the second level
 };
 
-enum SegFlags : uint32_t { SEG_LEVEL2 = 1u };
+enum SegFlags : uint32_t {
+  SEG_LEVEL2 = 1u,
+  SEG_SPEC = 2u  // k_lut predicts its active buckets (Candidates, below)
+};
+
+// Candidates.  Where a segment's ranks lie in few places (a top-K, a cluster,
+// a handful of ranks), k_lut predicts from the sample which buckets can hold
+// them, and the count pass, which reads every key anyway, also copies the
+// keys of those buckets into its chunk's part of the last eighth of the
+// segment's reduced buffer.  When every active bucket turns out to be one of
+// them (k_findk), the compaction reads a chunk's candidates in place of the
+// chunk: the second pass over the segment is gone.  A wrong prediction, a
+// chunk with more candidates than its part holds, or children that reach into
+// that eighth only bring the second pass back.  Measured (kernels of a select,
+// before and after): top-4096 of 2^28 floats 420 -> 276 us (compaction 161 ->
+// 8, count 168 -> 179), 256 ranks around the median and both extremes of 2^27
+// 248 -> 187 us (86 -> 9, 88 -> 103), a 4096-segment batch, half of it top-K,
+// 3948 -> 3438 us.  The share of buckets tried is where the copies still cost
+// the count pass less than half of what the second pass does; 512 ranks that
+// lie apart never fit in it (kSpecCells tells before anything is built: at
+// 2^16 samples a rank off the ends takes 1.2 % of the keys, so seven of them
+// fit, each touching two cells at most), and below 2^17 keys the second pass costs no more
+// than the prediction (2 us).
+constexpr uint32_t kSpecRanks = 512;   // most ranks of a multiselect tried
+constexpr uint32_t kSpecShare = 12;    // at most 1 / kSpecShare of the buckets
+constexpr uint32_t kSpecCells = 14;    // most 64ths of the vector with ranks in them
+constexpr uint32_t kSpecAreaLog2 = 3;  // candidates per chunk: len >> kSpecAreaLog2
+constexpr uint64_t kSpecMinLen = 1ull << 17;
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+// Start of a chunk's candidates in its segment's part of the reduced buffer
+// (chunk starts are multiples of 64 keys).
+inline uint64_t spec_area(uint64_t seg_len, uint64_t chunk_start) {
+  return seg_len - (seg_len >> kSpecAreaLog2) + (chunk_start >> kSpecAreaLog2);
+}
 
 // The bucket function of a segment (BucketFn in ggks_kernels.hpp):
 //   low = min(max(key, kb) - kb, lmax)      keys outside the sampled range
@@ -94,7 +129,9 @@ struct SegState {         // written on the device by the LUT kernel
   uint32_t hvon;          // 1: the heavy-value bucket is in use
   uint32_t hb;            // F's bucket of hv (L(hv) + 1) when hvon
   uint32_t nfree;         // next free child slot (second-level children)
-  uint32_t arrive;        // LUT parts done (k_lut; zeroed by k_sample)
+  uint32_t arrive;        // LUT parts done (k_lut; zeroed by k_sample); afterwards
+                          // 1: the count pass collects candidates (k_lut), the
+                          // compaction reads them (k_findk)
   uint32_t nred;          // keys of the active buckets (k_findk)
 };
 
