@@ -18,9 +18,8 @@
 //             rank's digit gathered and ranked (keys in registers when they
 //             fit); per child of up to 1024 keys with many ranks: its keys
 //             in LDS in the order of nearly even bins (bin_select)
-//   k_finish  every other child: bin_select when its keys fit LDS (a sort or
-//             8-bit digit passes where bins stay crowded), else multi-rank
-//             MSD radix select on 8-bit digits of (key - lo) from memory
+//   k_finish  every other child: bin_select when its keys fit LDS (a sort
+//             where bins stay crowded), else per run of its bins that does
 // Plans of at most 4096 buckets per segment run k_count_small, k_findk_small
 // and k_compact_small: the same bodies with smaller tables, two work-groups
 // per CU.  Plans whose children are small run k_finish_small_lite (4-byte keys):
@@ -512,8 +511,10 @@ struct RangeOf {
 };
 
 // Visit every element of p[0, len) with f(raw), 16-byte vector loads for the
-// aligned body, four loads in flight per thread.
-template <typename KT, typename F>
+// aligned body, D loads in flight per thread.  With TAIL the last, partial
+// round's loads are in flight together, too: what a work-group alone on its
+// child waits for is the number of rounds.
+template <uint32_t D = 4, bool TAIL = false, typename KT, typename F>
 __device__ __forceinline__ void for_each_elem(const KT* __restrict__ p, uint64_t len, F&& f) {
   constexpr uint32_t VEC = 16 / sizeof(KT);
   const uint32_t tid = threadIdx.x;
@@ -532,11 +533,26 @@ __device__ __forceinline__ void for_each_elem(const KT* __restrict__ p, uint64_t
       f((KT)(((uint64_t)v.w << 32) | v.z));
     }
   };
-  for (; i + 3 * kThreads < nvec; i += 4 * kThreads) {
-    uint4 a = pv[i], b = pv[i + kThreads], c = pv[i + 2 * kThreads], d = pv[i + 3 * kThreads];
-    apply(a); apply(b); apply(c); apply(d);
+  for (; i + (D - 1) * kThreads < nvec; i += D * kThreads) {
+    uint4 v[D];
+#pragma unroll
+    for (uint32_t u = 0; u < D; ++u) v[u] = pv[i + u * kThreads];
+#pragma unroll
+    for (uint32_t u = 0; u < D; ++u) apply(v[u]);
   }
-  for (; i < nvec; i += kThreads) apply(pv[i]);
+  if (TAIL) {
+    if (i < nvec) {
+      uint4 v[D];
+#pragma unroll
+      for (uint32_t u = 0; u < D; ++u)
+        if (i + u * kThreads < nvec) v[u] = pv[i + u * kThreads];
+#pragma unroll
+      for (uint32_t u = 0; u < D; ++u)
+        if (i + u * kThreads < nvec) apply(v[u]);
+    }
+  } else {
+    for (; i < nvec; i += kThreads) apply(pv[i]);
+  }
   const uint64_t done = head + nvec * VEC;
   if (done + tid < len) f(p[done + tid]);
 }
@@ -1654,12 +1670,10 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
     cp->q_cnt = next - first;
     const uint64_t clen = cp->len;
     // the key range where a later step needs it before reading the keys (a
-    // child the second level may take, or one k_finish walks from memory);
-    // a child of few ranks held in the 256-thread finisher's registers gets
-    // the exact min and max of its keys there, one pass over registers,
-    // which is cheaper than inverting the bucket function here
-    if ((l2 && clen > kHeavyKeys) || clen > finish_small_reg_keys<KT>(false) ||
-        next - first > kWaveRanks) {
+    // child the second level may take, or one that a finisher walks from
+    // memory); the others get the exact min and max of their keys in the
+    // finisher, which is cheaper than inverting the bucket function here
+    if ((l2 && clen > kHeavyKeys) || clen > finish_small_reg_keys<KT>(false)) {
       KT klo, khi;
       range(cp->bucket, klo, khi);
       cp->lo = klo;
@@ -2589,9 +2603,6 @@ __global__ __launch_bounds__(kThreads) void k_copy16(const uint4* __restrict__ s
     dst[i] = stream_load(&src[i]);
 }
 
-// k_finish sorts a child held in LDS when it has many ranks or is short
-// enough that a sort beats the digit passes.
-constexpr uint32_t kSortLen = 4096;
 constexpr uint32_t kFDigit = 11;                      // first digit: 2048 bins
 constexpr uint32_t kFWords = (1u << kFDigit) + (1u << kFDigit) / 32;  // padded: bin b at b + b/32
 constexpr uint32_t kFCollectWords = 1024;             // keys gathered after the first digit
@@ -2743,14 +2754,16 @@ __device__ __forceinline__ void wave_pick256(const uint32_t* h, uint32_t lane, u
 // 21 -> 14 us; a 4096-segment batch's children 472 -> 190 us.
 // Returns false (nothing lost: srt then holds the keys minus lo, in some
 // order) where the ranks of crowded bins would read more than kBinWork keys
-// in all; the caller then sorts or takes digit passes over the whole child.
+// in all; the caller then sorts the keys.
 constexpr uint32_t kBinThread = 8;
 constexpr uint32_t kBinWork = 1u << 16;
 template <uint32_t NT>
 constexpr uint32_t kFineBins = NT == kThreads ? 8192 : 4 * NT;
-template <typename KT, int C, uint32_t NT, uint32_t S>
+// The keys come from srcp, or (INLDS) from srt; answered are the queries of
+// ranks rank0 + 1 .. rank0 + len.
+template <typename KT, int C, uint32_t NT, uint32_t S, bool INLDS>
 __device__ bool bin_select(const KT* __restrict__ srcp, uint32_t len, const Query* __restrict__ cq,
-                           uint32_t q_cnt, KT* __restrict__ out, KT* srt, uint32_t* hist,
+                           uint32_t q_cnt, uint32_t rank0, KT* __restrict__ out, KT* srt, uint32_t* hist,
                            uint32_t* coarse, uint32_t* whist, uint4* list, KT* red_lo, KT* red_hi,
                            uint32_t* misc, KT& lo_out, int& nbits_out) {
   constexpr uint32_t NW = NT / 64, FB = kFineBins<NT>, WPT = FB / NT;  // fine bins per thread
@@ -2769,7 +2782,7 @@ __device__ bool bin_select(const KT* __restrict__ srcp, uint32_t len, const Quer
 #pragma unroll
   for (uint32_t t = 0; t < S; ++t) {
     const uint32_t i = t * NT + tid;
-    k[t] = i < len ? srcp[i] : KT(0);
+    k[t] = i < len ? (INLDS ? srt[i] : srcp[i]) : KT(0);
   }
   const Query q0 = tid < q_cnt ? cq[tid] : Query{1, 0};  // arrives with the keys
 #pragma unroll
@@ -2869,9 +2882,9 @@ __device__ bool bin_select(const KT* __restrict__ srcp, uint32_t len, const Quer
   nbits_out = nbits;
   for (uint32_t q1 = 0; q1 < q_cnt; q1 += NT) {  // uniform
     // one rank a thread; the crowded ones are listed (16 bytes each)
-    if (q1 + tid < q_cnt) {
-      const Query q = q1 == 0 ? q0 : cq[q1 + tid];
-      const uint32_t r = q.rank - 1;
+    const Query q = q1 + tid >= q_cnt ? Query{0, 0} : q1 == 0 ? q0 : cq[q1 + tid];
+    const uint32_t r = q.rank - 1 - rank0;
+    if (q1 + tid < q_cnt && r < len) {
       KT x = srt[r];
       const uint32_t e = coarse[(uint32_t)(x >> sh)];
       const uint32_t low = sh == 0 ? 0u : sh <= 32 ? (uint32_t)x << (32 - sh) : (uint32_t)(x >> (sh - 32));
@@ -3214,9 +3227,9 @@ __device__ __forceinline__ void finish_small_body(const KT* __restrict__ input,
       const uint32_t len = (uint32_t)c.len;
       KT lo;
       int nbits;
-      if (!bin_select<KT, C, kFThreads, kSortCap / kFThreads>(srcp, len, cq, c.q_cnt, out, keys, sbins,
-                                                              scoarse, swave, slist, red_lo, red_hi,
-                                                              smisc, lo, nbits)) {
+      if (!bin_select<KT, C, kFThreads, kSortCap / kFThreads, false>(
+              srcp, len, cq, c.q_cnt, 0u, out, keys, sbins, scoarse, swave, slist, red_lo, red_hi, smisc,
+              lo, nbits)) {
         uint32_t np = 1;
         while (np < len) np <<= 1;
         for (uint32_t i = len + tid; i < np; i += kFThreads) keys[i] = KeyBits<KT>::MAX;
@@ -3250,22 +3263,32 @@ __global__ __launch_bounds__(kFThreads) __attribute__((amdgpu_waves_per_eu(6))) 
 }
 #undef GGKS_FINISH_PARAMS
 
-// Finisher: exact multi-rank radix select inside each child.
-// LDS layout (byte offsets, all 16-aligned): keys | hist | queries | query
-// prefixes | group prefixes | min/max scratch | group starts | misc.
+// Finisher of every other child, a work-group of 1024 threads each: bin_select
+// where the keys fit LDS; where they do not, one histogram of the child over
+// 4096 bins of a window of its key range and, per run of bins that fits LDS
+// and holds ranks, one pass that gathers the run's keys for bin_select.
+// Ascending windows: the whole range, or a bin too long for LDS by itself.
+// Bound by one CU's passes over the child (about 8 us each for 50 K keys),
+// three of them where 8-bit digit passes over groups of 32 ranks took up to
+// hundreds: the 4096 largest of 2^28 uniform floats (a child of 60 K keys)
+// 1078 -> 295 us a select, of 2^26 floats of 1024 values 1196 -> 215 us, two
+// children of 37 K doubles with a few ranks each 96 -> 47 us.
+// LDS layout (byte offsets, all 16-aligned): keys | fine bins | list of ranks
+// in crowded bins | wavefront histograms | window bins | coarse bins | range
+// parts | misc | window bins with ranks | list of children.
+constexpr uint32_t kWideBits = 12, kWideBins = 1u << kWideBits;
 constexpr uint32_t kFinishOffHist = kFinishLdsBytes;
-constexpr uint32_t kFinishOffQv = kFinishOffHist + kGroupMax * 256 * 4;
-constexpr uint32_t kFinishOffQpre = kFinishOffQv + kQCap * 8;
-constexpr uint32_t kFinishOffGpre = kFinishOffQpre + kQCap * 8;
-constexpr uint32_t kFinishOffRed = kFinishOffGpre + (kGroupMax + 2) * 8;
-constexpr uint32_t kFinishOffGfirst = kFinishOffRed + 32 * 8;
-constexpr uint32_t kFinishOffMisc = kFinishOffGfirst + ((kQCap + 1) * 4 + 15) / 16 * 16;
-constexpr uint32_t kFinishOffList = kFinishOffMisc + 32 * 4;
-constexpr uint32_t kFinishOffWave = (kFinishOffList + (kThreads + 4) * 4 + 15) / 16 * 16;
-constexpr uint32_t kFinishLdsTotal = kFinishOffWave + kThreads / 64 * 256 * 4;
-static_assert(kGroupMax * 256 >= kFineBins<kThreads> && kQCap >= kThreads, "bin_select's bins fit");
-static_assert(kThreads <= kQCap, "bin_select's list fits the query arrays");
+constexpr uint32_t kFinishOffRanks = kFinishOffHist + kFineBins<kThreads> * 4;
+constexpr uint32_t kFinishOffWave = kFinishOffRanks + kThreads * 16;
+constexpr uint32_t kFinishOffWide = kFinishOffWave + kThreads / 64 * 256 * 4;
+constexpr uint32_t kFinishOffCoarse = kFinishOffWide + kWideBins * 4;
+constexpr uint32_t kFinishOffRed = kFinishOffCoarse + kThreads * 4;
+constexpr uint32_t kFinishOffMisc = kFinishOffRed + 32 * 8;
+constexpr uint32_t kFinishOffNeed = kFinishOffMisc + 32 * 4;
+constexpr uint32_t kFinishOffList = kFinishOffNeed + kWideBins / 32 * 4;
+constexpr uint32_t kFinishLdsTotal = kFinishOffList + (kThreads + 4) * 4;
 static_assert(kThreads / 64 + 2 <= 32, "bin_select's totals fit the misc words");
+static_assert(kFinishLdsTotal <= 160 * 1024, "LDS of the finisher");
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ input,
                                                      const KT* __restrict__ red,
@@ -3278,23 +3301,21 @@ __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ inpu
                                                      const uint32_t* __restrict__ bigw) {
   // nothing to do when k_findk counted no child for this finisher
   if (bigw && *bigw == 0) return;  // uniform
-  constexpr uint32_t W = KeyBits<KT>::W;
-  constexpr uint32_t CAP = kFinishLdsBytes / sizeof(KT);
+  constexpr uint32_t CAP = kFinishLdsBytes / sizeof(KT), S = CAP / kThreads;
   extern __shared__ __align__(16) uint32_t lds[];
   char* base = reinterpret_cast<char*>(lds);
   KT* keys = reinterpret_cast<KT*>(base);
   uint32_t* hist = reinterpret_cast<uint32_t*>(base + kFinishOffHist);
-  uint64_t* qv = reinterpret_cast<uint64_t*>(base + kFinishOffQv);  // (rank << 32) | out
-  KT* qpre = reinterpret_cast<KT*>(base + kFinishOffQpre);           // relative prefix
-  KT* gpre = reinterpret_cast<KT*>(base + kFinishOffGpre);           // group prefixes
-  KT* red_lo = reinterpret_cast<KT*>(base + kFinishOffRed);          // 16
-  KT* red_hi = red_lo + 16;                                          // 16
-  uint32_t* gfirst = reinterpret_cast<uint32_t*>(base + kFinishOffGfirst);  // kQCap + 1
-  uint32_t* misc = reinterpret_cast<uint32_t*>(base + kFinishOffMisc);      // 32 words
-  uint32_t* list = reinterpret_cast<uint32_t*>(base + kFinishOffList);      // kThreads + count
+  uint4* ranks = reinterpret_cast<uint4*>(base + kFinishOffRanks);
+  uint32_t* whist = reinterpret_cast<uint32_t*>(base + kFinishOffWave);  // 256 a wavefront
+  uint32_t* wide = reinterpret_cast<uint32_t*>(base + kFinishOffWide);
+  uint32_t* coarse = reinterpret_cast<uint32_t*>(base + kFinishOffCoarse);
+  KT* red_lo = reinterpret_cast<KT*>(base + kFinishOffRed);  // 16
+  KT* red_hi = red_lo + 16;                                  // 16
+  uint32_t* misc = reinterpret_cast<uint32_t*>(base + kFinishOffMisc);  // 32 words
+  uint32_t* need = reinterpret_cast<uint32_t*>(base + kFinishOffNeed);
+  uint32_t* list = reinterpret_cast<uint32_t*>(base + kFinishOffList);  // kThreads + count
   uint32_t& nlist = list[kThreads];
-  uint32_t* whist = reinterpret_cast<uint32_t*>(base + kFinishOffWave);     // 256 a wavefront
-  uint4* blist = reinterpret_cast<uint4*>(qv);                              // qv and qpre
   const uint32_t tid = threadIdx.x;
 
   // this work-group's children are blockIdx.x, + gridDim.x, ...; they are
@@ -3316,159 +3337,167 @@ __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ inpu
     for (uint32_t li = 0; li < nl; ++li) {
       const Child c = children[list[li]];
       const KT* srcp = (c.src == 0 ? input : (c.src == 1 ? red : red2)) + c.start;
-      const Query* __restrict__ cq = c.src == 2 ? cq2 : cq0;
-      const bool inl = c.len <= CAP;
-      KT lo = (KT)c.lo, hi = (KT)c.hi;
-      int nbits;
-      if (inl) {
-        if (bin_select<KT, C, kThreads, CAP / kThreads>(srcp, (uint32_t)c.len, cq + c.q_off, c.q_cnt,
-                                                        out, keys, hist, gfirst, whist, blist,
-                                                        red_lo, red_hi, misc, lo, nbits)) {
-          __syncthreads();
-          continue;
+      const Query* __restrict__ cq = (c.src == 2 ? cq2 : cq0) + c.q_off;
+      // the ranks rank0 + 1 .. rank0 + len from keys (crowded bins under many
+      // ranks: n keys minus lo, in any order), sorted: every rank is a look-up
+      auto sorted = [&](uint32_t len, uint32_t rank0, KT lo, int nbits) {
+        const uint32_t np = (len + kThreads - 1) / kThreads * kThreads;
+        for (uint32_t i = len + tid; i < np; i += kThreads) keys[i] = KeyBits<KT>::MAX;
+        __syncthreads();
+        lds_radix_sort<KT, S>(keys, np, nbits, hist, misc);
+        for (uint32_t i = tid; i < c.q_cnt; i += kThreads) {
+          const Query q = cq[i];
+          const uint32_t r = q.rank - 1 - rank0;
+          if (r < len) out[q.out] = from_key<C>((KT)(lo + keys[r]));
         }
-        // crowded bins under many ranks; keys holds the child minus lo
-        if (c.q_cnt > kSortRanks || c.len <= kSortLen) {
-          // sort the keys in LDS, then every rank is a lookup
-          const uint32_t np = ((uint32_t)c.len + kThreads - 1) / kThreads * kThreads;
-          for (uint32_t i = c.len + tid; i < np; i += kThreads) keys[i] = KeyBits<KT>::MAX;
-          __syncthreads();
-          lds_radix_sort<KT, CAP / kThreads>(keys, np, nbits, hist, misc);
-          for (uint32_t i = tid; i < c.q_cnt; i += kThreads) {
-            Query q = cq[c.q_off + i];
-            out[q.out] = from_key<C>((KT)(lo + keys[q.rank - 1]));
-          }
-          __syncthreads();
-          continue;
+      };
+      if (c.len <= CAP) {
+        KT lo;
+        int nbits;
+        if (!bin_select<KT, C, kThreads, S, false>(srcp, (uint32_t)c.len, cq, c.q_cnt, 0u, out, keys,
+                                                   hist, coarse, whist, ranks, red_lo, red_hi, misc,
+                                                   lo, nbits))
+          sorted((uint32_t)c.len, 0u, lo, nbits);
+        __syncthreads();
+        continue;
+      }
+      // the keys' range: their bucket's or digit's, or their own (a direct
+      // child's)
+      KT wlo = (KT)c.lo, hi = (KT)c.hi;
+      if (c.need_range) {
+        KT a = KeyBits<KT>::MAX, b = 0;
+        for_each_elem<8, true>(srcp, c.len, [&](KT raw) {
+          const KT k = to_key<C>(raw);
+          a = k < a ? k : a;
+          b = k > b ? k : b;
+        });
+        for (int d = 32; d >= 1; d >>= 1) {
+          KT x = __shfl_xor(a, d, 64), y = __shfl_xor(b, d, 64);
+          a = x < a ? x : a;
+          b = y > b ? y : b;
         }
-      } else {
-        if (c.need_range) {
-          KT a = KeyBits<KT>::MAX, b = 0;
-          for_each_elem(srcp, c.len, [&](KT raw) {  // 16-byte loads, four in flight per thread
-            const KT k = to_key<C>(raw);
-            a = k < a ? k : a;
-            b = k > b ? k : b;
+        if (lane_id() == 0) { red_lo[tid >> 6] = a; red_hi[tid >> 6] = b; }
+        __syncthreads();
+        wlo = red_lo[0]; hi = red_hi[0];
+        for (int w = 1; w < 16; ++w) {
+          wlo = red_lo[w] < wlo ? red_lo[w] : wlo;
+          hi = red_hi[w] > hi ? red_hi[w] : hi;
+        }
+      }
+      KT whi = hi;         // the window [wlo, whi]
+      uint32_t below = 0;  // the child's keys below it
+      bool whole = true;   // no key lies outside it
+      for (;;) {
+        const int nbits = bitlen<KT>((KT)(whi - wlo));
+        const int sh = nbits > (int)kWideBits ? nbits - (int)kWideBits : 0;
+        __syncthreads();  // the last window's words are read
+        for (uint32_t i = tid; i < kWideBins; i += kThreads) wide[i] = 0;
+        if (tid < kWideBins / 32) need[tid] = 0;
+        __syncthreads();
+        if (whole)  // uniform
+          for_each_elem<8, true>(srcp, c.len, [&](KT raw) {
+            atomicAdd(&wide[(uint32_t)((KT)(to_key<C>(raw) - wlo) >> sh)], 1u);
           });
-          for (int d = 32; d >= 1; d >>= 1) {
-            KT x = __shfl_xor(a, d, 64), y = __shfl_xor(b, d, 64);
-            a = x < a ? x : a;
-            b = y > b ? y : b;
-          }
-          if (lane_id() == 0) { red_lo[tid >> 6] = a; red_hi[tid >> 6] = b; }
-          __syncthreads();
-          lo = red_lo[0]; hi = red_hi[0];
-          for (int w = 1; w < 16; ++w) {
-            lo = red_lo[w] < lo ? red_lo[w] : lo;
-            hi = red_hi[w] > hi ? red_hi[w] : hi;
+        else
+          for_each_elem<8, true>(srcp, c.len, [&](KT raw) {
+            const KT k = to_key<C>(raw);
+            if (k >= wlo && k <= whi) atomicAdd(&wide[(uint32_t)((KT)(k - wlo) >> sh)], 1u);
+          });
+        __syncthreads();
+        const uint32_t total = block_scan_array(wide, kWideBins, misc);  // (synchronises)
+        auto end_of = [&](uint32_t b) { return b + 1 < kWideBins ? wide[b + 1] : total; };
+        for (uint32_t i = tid; i < c.q_cnt; i += kThreads) {
+          const Query q = cq[i];
+          const uint32_t r = q.rank - 1 - below;
+          if (r < total) {
+            uint32_t a = 0, z = kWideBins - 1;  // largest bin with start <= r
+            while (a < z) {
+              const uint32_t m = (a + z + 1) >> 1;
+              if (wide[m] <= r) a = m; else z = m - 1;
+            }
+            if (sh == 0) out[q.out] = from_key<C>((KT)(wlo + a));  // a bin is a value
+            else lds_or(need, a >> 5, 1u << (a & 31u));
           }
         }
-        nbits = bitlen<KT>(hi - lo);
+        __syncthreads();
+        // the first, or last, bin of [a, z] with ranks; kWideBins: none
+        auto marked = [&](uint32_t a, uint32_t z, bool last) -> uint32_t {
+          static_assert(kWideBins == 128 * 32, "two words a lane");
+          uint32_t m[2];
+#pragma unroll
+          for (uint32_t h = 0; h < 2; ++h) {
+            const uint32_t w = h * 64 + lane_id();
+            m[h] = w < (a >> 5) || w > (z >> 5) ? 0u : need[w];
+            if (w == a >> 5) m[h] &= ~0u << (a & 31u);
+            if (w == z >> 5) m[h] &= ~0u >> (31u - (z & 31u));
+          }
+          const uint64_t k0 = __ballot(m[0] != 0), k1 = __ballot(m[1] != 0);
+          if (!(k0 | k1)) return kWideBins;
+          const bool high = last ? k1 != 0 : k0 == 0;
+          const uint64_t k = high ? k1 : k0;
+          const uint32_t l = last ? 63u - (uint32_t)__clzll((long long)k)
+                                  : (uint32_t)__ffsll((unsigned long long)k) - 1u;
+          const uint32_t word = wave_lane<uint32_t>(high ? m[1] : m[0], l);
+          return ((high ? 64u : 0u) + l) * 32u +
+                 (last ? 31u - (uint32_t)__clz((int)word) : (uint32_t)__ffs(word) - 1u);
+        };
+        bool narrowed = false;
+        for (uint32_t pos = 0; pos < kWideBins;) {  // uniform
+          // the first bin with ranks from pos on (every wavefront finds it)
+          const uint32_t b0 = marked(pos, kWideBins - 1, false);
+          if (b0 == kWideBins) break;
+          const uint32_t s0 = wide[b0];
+          if (end_of(b0) - s0 > CAP) {  // too long by itself: its range is the next window
+            wlo = (KT)(wlo + ((KT)b0 << sh));
+            const KT w = (KT)((KT(1) << sh) - 1);
+            whi = (KT)(whi - wlo) > w ? (KT)(wlo + w) : whi;
+            below += s0;
+            narrowed = true;
+            whole = false;
+            break;
+          }
+          uint32_t b1 = b0, z = kWideBins - 1;  // the last bin of the run that fits
+          while (b1 < z) {
+            const uint32_t m = (b1 + z + 1) >> 1;
+            if (end_of(m) - s0 <= CAP) b1 = m; else z = m - 1;
+          }
+          b1 = marked(b0, b1, true);  // and holds ranks (b0 does)
+          const uint32_t n = end_of(b1) - s0;
+          __syncthreads();  // keys of the last run are read
+          if (tid == 0) misc[24] = 0;
+          __syncthreads();
+          // (keys of the bins b0 .. b1 are those from klo to klo + kspan; a
+          // whole window's last bin may reach past it)
+          const KT klo = (KT)(wlo + ((KT)b0 << sh));
+          KT kspan = (KT)(((KT)(b1 - b0 + 1) << sh) - 1);
+          kspan = (KT)(whi - klo) < kspan ? (KT)(whi - klo) : kspan;
+          for_each_elem<8, true>(srcp, c.len, [&](KT raw) {
+            const bool in = (KT)(to_key<C>(raw) - klo) <= kspan;
+            const uint64_t m = __ballot(in);
+            if (in) {  // one atomic a wavefront
+              const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+              uint32_t first = 0;
+              if (at == 0) first = atomicAdd(&misc[24], (uint32_t)__popcll(m));
+              first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+              keys[first + at] = raw;
+            }
+          });
+          __syncthreads();
+          KT lo;
+          int nb;
+          if (!bin_select<KT, C, kThreads, S, true>(keys, n, cq, c.q_cnt, below + s0, out, keys, hist,
+                                                    coarse, whist, ranks, red_lo, red_hi, misc, lo, nb))
+            sorted(n, below + s0, lo, nb);
+          pos = b1 + 1;
+        }
+        if (narrowed) continue;
+        if (whi == hi) break;
+        below += total;
+        wlo = (KT)(whi + 1);
+        whi = hi;
       }
       __syncthreads();
-
-      for (uint32_t q0 = 0; q0 < c.q_cnt; q0 += kQCap) {
-        const uint32_t nq = min(kQCap, c.q_cnt - q0);
-        // queries sorted by rank: bitonic sort of the padded power of two
-        uint32_t np = 1;
-        while (np < nq) np <<= 1;
-        for (uint32_t i = tid; i < np; i += kThreads) {
-          if (i < nq) {
-            Query q = cq[c.q_off + q0 + i];
-            qv[i] = ((uint64_t)q.rank << 32) | q.out;
-          } else {
-            qv[i] = ~0ull;
-          }
-        }
-        __syncthreads();
-        lds_bitonic_sort<kThreads, (kQCap / 2 + kThreads - 1) / kThreads>(qv, np);
-        for (uint32_t i = tid; i < nq; i += kThreads) qpre[i] = 0;
-        __syncthreads();
-
-        // digit levels from the top of the relative range
-        int rem = nbits;
-        while (rem > 0) {
-          const int d = rem < 8 ? rem : 8;
-          const int shift = rem - d;
-          const int hshift = shift + d;  // bits above the digit
-          // groups = runs of equal prefix (queries are rank-sorted, so prefixes
-          // are non-decreasing)
-          if (tid == 0) {
-            uint32_t g = 0;
-            for (uint32_t i = 0; i < nq; ++i)
-              if (i == 0 || qpre[i] != qpre[i - 1]) gfirst[g++] = i;
-            gfirst[g] = nq;
-            misc[0] = g;
-          }
-          __syncthreads();
-          const uint32_t ng = misc[0];
-          for (uint32_t g0 = 0; g0 < ng; g0 += kGroupMax) {
-            const uint32_t gn = min(kGroupMax, ng - g0);
-            for (uint32_t i = tid; i < gn * 256; i += kThreads) hist[i] = 0;
-            for (uint32_t g = tid; g < gn; g += kThreads) gpre[g] = qpre[gfirst[g0 + g]];
-            __syncthreads();
-            auto visit = [&](KT rel) {
-              KT pre = hshift >= (int)W ? KT(0) : (rel >> hshift);
-              uint32_t g;
-              if (gn == 1) {
-                if (pre != gpre[0]) return;
-                g = 0;
-              } else {
-                uint32_t a = 0, b = gn - 1;
-                while (a < b) {
-                  uint32_t mid = (a + b) >> 1;
-                  if (gpre[mid] < pre) a = mid + 1; else b = mid;
-                }
-                if (gpre[a] != pre) return;
-                g = a;
-              }
-              atomicAdd(&hist[g * 256 + (uint32_t)((rel >> shift) & (KT)((1u << d) - 1))], 1u);
-            };
-            if (inl) {
-              for (uint32_t i = tid; i < c.len; i += kThreads) visit(keys[i]);
-            } else {  // 16-byte loads, four in flight per thread
-              for_each_elem(srcp, c.len, [&](KT raw) { visit((KT)(to_key<C>(raw) - lo)); });
-            }
-            __syncthreads();
-            // exclusive scan of each group's 256 bins: one wave per group
-            const uint32_t wv = tid >> 6, lane = lane_id();
-            for (uint32_t g = wv; g < gn; g += kThreads / 64) {
-              uint32_t* h = hist + g * 256;
-              uint32_t v0 = h[lane * 4], v1 = h[lane * 4 + 1], v2 = h[lane * 4 + 2], v3 = h[lane * 4 + 3];
-              uint32_t s = v0 + v1 + v2 + v3;
-              uint32_t e = wave_incl_scan(s) - s;
-              h[lane * 4] = e;
-              h[lane * 4 + 1] = e + v0;
-              h[lane * 4 + 2] = e + v0 + v1;
-              h[lane * 4 + 3] = e + v0 + v1 + v2;
-            }
-            __syncthreads();
-            // every query of these groups picks its digit
-            const uint32_t qa = gfirst[g0], qz = gfirst[g0 + gn];
-            for (uint32_t i = qa + tid; i < qz; i += kThreads) {
-              uint32_t a = 0, b = gn - 1;  // group of query i
-              while (a < b) {
-                uint32_t mid = (a + b + 1) >> 1;
-                if (gfirst[g0 + mid] <= i) a = mid; else b = mid - 1;
-              }
-              const uint32_t* h = hist + a * 256;
-              uint32_t r1 = (uint32_t)(qv[i] >> 32) - 1;
-              uint32_t lo_d = 0, hi_d = (1u << d) - 1;  // largest digit with h <= r1
-              while (lo_d < hi_d) {
-                uint32_t mid = (lo_d + hi_d + 1) >> 1;
-                if (h[mid] <= r1) lo_d = mid; else hi_d = mid - 1;
-              }
-              uint32_t nr = r1 - h[lo_d] + 1;
-              qv[i] = ((uint64_t)nr << 32) | (uint32_t)qv[i];
-              qpre[i] = (qpre[i] << d) | (KT)lo_d;
-            }
-            __syncthreads();
-          }
-          rem = shift;
-        }
-        for (uint32_t i = tid; i < nq; i += kThreads)
-          out[(uint32_t)qv[i]] = from_key<C>((KT)(lo + qpre[i]));
-        __syncthreads();
-      }
     }
     __syncthreads();  // every thread is done with the list before it is refilled
   }

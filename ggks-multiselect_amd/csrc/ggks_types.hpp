@@ -16,10 +16,7 @@ constexpr uint32_t kMaxBuckets = 32768;    // histogram bins per segment (LDS)
 constexpr uint32_t kMaxPrefixBits = 12;    // LUT prefixes per segment <= 4096
 constexpr uint32_t kCursorCap = 4096;      // LDS write cursors in compaction
 constexpr uint32_t kFinishLdsBytes = 65536;// keys kept in LDS by the finisher
-constexpr uint32_t kQCap = 1024;           // queries per finisher batch
-constexpr uint32_t kGroupMax = 32;         // prefix groups per histogram pass
 constexpr uint32_t kReduceBins = 64;       // bins per reduce work item
-constexpr uint32_t kSortRanks = 32;        // finisher sorts a child above this
 constexpr uint32_t kMaxChunks = 512;       // chunks per segment (reduce registers)
 
 // Where a segment's queries come from.

@@ -4,7 +4,7 @@ threads), 64 KB of keys (1024 threads) and one key past each; a few ranks,
 one more than a work-group takes at a time, and every rank; keys spread
 evenly, crowded at one end of their range, around zero, in copies of few
 values (crowded bins: a wavefront each), in copies of one, and a few bins
-holding everything (the sort and the digit passes behind it)."""
+holding everything (the sort behind it)."""
 import numpy as np
 import pytest
 
@@ -46,4 +46,35 @@ def test_many_ranks_of_one_child(pkg, O, dtype, fam):
             got = pkg.topk(d, nk, ctx)
             assert np.array_equal(bits(got), bits(O.topk(x, nk))), (n, nk)
         d.free()
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.uint32, np.int32])
+@pytest.mark.parametrize("fam", ["lump", "copies", "zero"])
+def test_ranks_of_a_child_past_lds(pkg, O, dtype, fam):
+    """A child longer than 64 KB of keys, finished window by window: most
+    keys in one bucket, spread out in it, in copies of a few values (bins
+    longer than LDS, bins that are one value), or around zero (floats crowd
+    at both ends of the bucket); one rank, a few, and more than one round of
+    them, clustered and spread."""
+    W = pkg.workloads
+    ctx = pkg.Context(0)
+    n = 150_001
+    if fam == "copies":
+        x = (W.uint_range(6, n, 0, 6).astype(np.int64) * 3 + (W.uint_range(7, n, 0, 99) == 0)).astype(dtype)
+    elif fam == "lump" or np.dtype(dtype).kind != "f":
+        x = (W.uint_range(6, n, 0, 1 << 18).astype(np.int64) + 5000).astype(dtype)
+    else:
+        x = (W.normal_f64(6, n) * 1e-20).astype(dtype) + 0
+    x[:300] = (np.arange(300, dtype=np.int64) * 7_000_000).astype(dtype)  # the range around the lump
+    d = pkg.DeviceArray.from_host(x)
+    for k in ([n // 2], [1, 2, n // 3, n // 2, n // 2 + 1, n], np.arange(n // 2, n // 2 + 700),
+              W.k_uniform(8, n, 2500, dedup=False)):
+        k = np.asarray(k, np.uint32)
+        print(f"past LDS {np.dtype(dtype).name} {fam} {k.size} k", flush=True)
+        got = pkg.multiselect(d, k, ctx, buckets_log2=8, level2=-1)
+        assert np.array_equal(bits(got), bits(O.sort_choose(x, k))), k.size
+        got = pkg.topk(d, k.size, ctx, buckets_log2=8, level2=-1)
+        assert np.array_equal(bits(got), bits(O.topk(x, k.size))), k.size
+    d.free()
     ctx.close()
