@@ -16,20 +16,57 @@ namespace ggks {
 
 inline size_t align_up(size_t x, size_t a = 256) { return (x + a - 1) / a * a; }
 
-// Tuned defaults per length band (bucket budget and chunk count).  The bucket
-// budget trades the reduced-set size (~ ranks * n / buckets) against the
-// per-chunk histogram rows (chunks * buckets * 4 bytes).
+// Tuned defaults per key width and length band (bucket budget and chunk
+// count).  The bucket budget trades the reduced-set size (~ ranks * n /
+// buckets) against the per-chunk histogram rows (chunks * buckets * 4 bytes),
+// which k_reduce and k_findk read in whole; a chunk per CU from 2^21 keys on.
+// Doubles take a bucket bit more than floats where their 11 exponent bits
+// leave the LUT's prefixes two or more binades wide (prefix bits = budget
+// bits - 2, at most 12).  Measured with 4 to 1000 ranks over normal, Cauchy
+// and uniform keys (us a select, before and after): 4e5 doubles 1000 ranks
+// 151 -> 59, 3e6 doubles 256 ranks 167 -> 69, 3e6 floats 64 -> 52, 8e5 floats
+// 1000 ranks 75 -> 54, 4e7 doubles 100 ranks 216 -> 167.
 struct Tuning {
   uint32_t buckets_log2;
   uint32_t chunks;
+  bool set;  // set by the caller (ggks_tuning_single_set): taken as it is
 };
 
-inline Tuning default_tuning(uint64_t n) {
-  if (n >= (1ull << 26)) return {15, 256};
-  if (n >= (1ull << 24)) return {13, 256};
-  if (n >= (1ull << 22)) return {12, 128};
-  if (n >= (1ull << 20)) return {11, 64};
-  return {10, 32};
+inline Tuning default_tuning(int key_bytes, int band) {
+  if (band >= 26) return {15, 256, false};
+  if (key_bytes == 8) {
+    if (band >= 24) return {14, 256, false};
+    if (band >= 22) return {13, 256, false};
+    if (band >= 20) return {12, 256, false};
+    if (band >= 18) return {12, 128, false};
+    if (band >= 16) return {12, 64, false};
+    return {11, 32, false};
+  }
+  if (band >= 24) return {13, 256, false};
+  if (band == 23) return {12, 256, false};
+  if (band == 22) return {12, 128, false};
+  if (band == 21) return {12, 256, false};
+  if (band >= 18) return {11, 128, false};
+  if (band >= 16) return {11, 64, false};
+  return {10, 32, false};
+}
+
+// The default budget of a select with few ranks (or a top-K, whose ranks lie
+// together): smaller tables, longer children.  The lines lie where the other
+// side measured slower on some of the distributions above (2^26 floats, 8 and
+// 100 ranks: 158 -> 138 and 153 -> 139 us with 2^13 buckets, 256 spread ranks
+// 156 -> 150 with 2^14; 2^28 floats, top-100: 247 -> 220 with 2^13).
+inline uint32_t few_ranks_log2(int key_bytes, int band, uint32_t nq, bool topk, uint32_t base) {
+  if (band >= 27) return topk ? 13 : nq <= (key_bytes == 8 ? 64u : 512u) ? 14 : base;
+  if (band == 26) return topk || nq <= (key_bytes == 8 ? 16u : 128u) ? 13 : nq <= 512 ? 14 : base;
+  if (key_bytes == 8) {
+    if (band >= 24) return topk || nq <= 128 ? 13 : base;
+    if (band >= 22) return topk || nq <= 16 ? 12 : base;
+    return base;
+  }
+  if (band >= 24) return topk || nq <= 64 ? 12 : base;
+  if (band == 21) return topk || nq <= 128 ? 11 : base;
+  return base;
 }
 
 // Single-vector tuning per (dtype, floor(log2 n)): the defaults above until
@@ -39,17 +76,19 @@ struct SingleTuningTable {
   Tuning t[4][kSingleBands];
   SingleTuningTable() {
     for (int d = 0; d < 4; ++d)
-      for (int b = 0; b < kSingleBands; ++b) t[d][b] = default_tuning(1ull << b);
+      for (int b = 0; b < kSingleBands; ++b) t[d][b] = default_tuning(dtype_bytes(d), b);
   }
 };
 inline SingleTuningTable& single_tuning_table() {
   static SingleTuningTable tab;
   return tab;
 }
-inline Tuning single_tuning(int dtype, uint64_t n) {
+inline Tuning single_tuning(int dtype, uint64_t n, uint32_t nq, bool topk) {
   int b = 0;
   while (b < kSingleBands - 1 && (n >> (b + 1))) ++b;
-  return single_tuning_table().t[dtype][b];
+  Tuning t = single_tuning_table().t[dtype][b];
+  if (!t.set) t.buckets_log2 = few_ranks_log2(dtype_bytes(dtype), b, nq, topk, t.buckets_log2);
+  return t;
 }
 
 // Bucket budget (log2) of a radix segment with digits of rb bits: room for
@@ -169,7 +208,7 @@ struct SingleShape {
   uint64_t G, csz;    // chunks and chunk length
 };
 
-inline SingleShape single_shape(int kind, int dtype, uint64_t n, const ggks_opts& o) {
+inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, const ggks_opts& o) {
   SingleShape sh = {};
   const int eb = dtype_bytes(dtype);
   const uint64_t cap = kFinishLdsBytes / (uint32_t)eb;
@@ -177,7 +216,7 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, const ggks_opts
     sh.direct = true;
     return sh;
   }
-  Tuning t = single_tuning(dtype, n);
+  const Tuning t = single_tuning(dtype, n, nq, kind == GGKS_KIND_TOPK);
   uint32_t bl;
   sh.mode = MODE_SAMPLE;
   if (kind == GGKS_KIND_RADIX) {
@@ -254,7 +293,7 @@ inline Child single_direct_child(uint64_t n, uint32_t nq) {
 inline void plan_single(Plan& p, int kind, int dtype, uint64_t n, uint32_t nq,
                         const ggks_opts& o, bool tables = true) {
   const int eb = dtype_bytes(dtype);
-  const SingleShape sh = single_shape(kind, dtype, n, o);
+  const SingleShape sh = single_shape(kind, dtype, n, nq, o);
   p.nq = nq;
   p.qmax = nq;
   p.seed = o.seed ? o.seed : 0x6A09E667F3BCC909ull;

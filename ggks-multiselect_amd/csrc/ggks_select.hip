@@ -749,6 +749,13 @@ static int select_noalloc(int dtype, const void* d_vec, int64_t n, const uint32_
   if (opt) o = *opt;
   Plan p;  // layout only: its table vectors stay empty
   plan_single(p, GGKS_KIND_BUCKET, dtype, (uint64_t)n, (uint32_t)num_k, o, false);
+  if (align_up(p.total) + 256 > kNoAllocScratchBytes) {
+    // near the limit: smaller histogram rows than the fastest shape's
+    if (!o.buckets_log2) o.buckets_log2 = 12;
+    if (!o.blocks) o.blocks = 128;
+    p = Plan();
+    plan_single(p, GGKS_KIND_BUCKET, dtype, (uint64_t)n, (uint32_t)num_k, o, false);
+  }
   const size_t off_status = align_up(p.total);
   const size_t need = off_status + 256;
   if (need > kNoAllocScratchBytes)
@@ -759,7 +766,7 @@ static int select_noalloc(int dtype, const void* d_vec, int64_t n, const uint32_
                 kNoAllocScratchBytes);
   char* base = nullptr;
   if ((rc = noalloc_base(&base))) return rc;
-  const SingleShape sh = single_shape(GGKS_KIND_BUCKET, dtype, (uint64_t)n, o);
+  const SingleShape sh = single_shape(GGKS_KIND_BUCKET, dtype, (uint64_t)n, (uint32_t)num_k, o);
   SinglePlanArgs a = {};
   a.n = (uint64_t)n;
   a.direct = p.direct ? 1u : 0u;
@@ -1159,7 +1166,7 @@ int ggks_tuning_single_set(int dtype, int log2_len, int buckets_log2, int chunks
   if (buckets_log2 < 8 || buckets_log2 > 15 || chunks < 1 || chunks > (int)kMaxChunks)
     return fail(GGKS_EINVAL, "bad single-vector tuning (buckets 2^%d, %d chunks)", buckets_log2,
                 chunks);
-  single_tuning_table().t[dtype][log2_len] = {(uint32_t)buckets_log2, (uint32_t)chunks};
+  single_tuning_table().t[dtype][log2_len] = {(uint32_t)buckets_log2, (uint32_t)chunks, true};
   return GGKS_OK;
 }
 
