@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(const KT* __restrict_
   const SampleBlock sb = sblocks[blockIdx.x];
   const SegDesc& sd = segs[sb.seg];
   if (sd.mode == MODE_RANGE || sb.blk * kThreads >= sd.nsample) return;  // uniform
-  if (sb.blk == 0 && lut_parts(sd.mode, sd.nsample, sizeof(KT)) > 1) {
+  if (sb.blk == 0 && lut_parts(seg_sampled(sd), sd.nsample, sizeof(KT)) > 1) {
     // the split LUT build adds its partial sample histograms into the LUT
     // region and counts its parts in the state: both start at zero
     for (uint32_t i = threadIdx.x; i < (1u << sd.pbits); i += kSampleThreads) lut_pool[sd.lut_off + i] = 0;
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample(const KT* __restrict_
   // the top bit (full-width ranges, such as floats of both signs) the LUT's
   // prefixes are exactly these bins, and k_lut reads 2^pbits counts instead
   // of histogramming the whole sample on one CU.
-  const bool hg = hgram != nullptr && sd.mode == MODE_SAMPLE;  // uniform
+  const bool hg = hgram != nullptr && seg_sampled(sd);  // uniform
   const uint32_t hsh = KeyBits<KT>::W - sd.pbits;
   if (hg)  // zeroed while the gathers are in flight
     for (uint32_t i = threadIdx.x; i < (1u << sd.pbits); i += kSampleThreads) hl[i] = 0;
@@ -849,6 +849,8 @@ __device__ __forceinline__ void predict(const uint32_t* cum, const uint32_t* ent
 //               RadixSelect_api.h:590-592, are skipped up front), each
 //               digit value exactly its buckets; keys outside the sampled
 //               window fall into a guard bucket below or above every digit.
+//               With SEG_REFINE a digit is cut further in proportion to its
+//               share of the sample, as MODE_SAMPLE's prefixes are.
 //  MODE_RANGE   equal-width buckets over the segment's known key range.
 // A heavy value of the sample (SegState) takes two more buckets.
 template <typename KT>
@@ -886,11 +888,11 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   const uint32_t myk = spec_k && tid < sd.q_cnt ? kraw[sd.q_off + tid] : 0u;
   // k_sample's prefix counts, loaded now (16 bytes a thread) so that they
   // arrive while the sample's range is reduced; used for full-width ranges
-  const bool hload = hgram && sd.mode == MODE_SAMPLE && tid < (1u << sd.pbits) / 4;
+  const bool hload = hgram && seg_sampled(sd) && tid < (1u << sd.pbits) / 4;
   const uint4 h4 = hload ? reinterpret_cast<const uint4*>(hgram)[tid] : make_uint4(0, 0, 0, 0);
   // part blockIdx.y of the segment's LUT build: its parts, at most the
   // grid's y extent (1 keeps every segment's build in one work-group)
-  const uint32_t nparts = min(lut_parts(sd.mode, sd.nsample, sizeof(KT)), gridDim.y), part = blockIdx.y;
+  const uint32_t nparts = min(lut_parts(seg_sampled(sd), sd.nsample, sizeof(KT)), gridDim.y), part = blockIdx.y;
   if (part >= nparts) return;  // uniform
   uint32_t* lut = lut_pool + sd.lut_off;
   if (tid < 2) sh_cells[tid] = 0;
@@ -949,10 +951,15 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   // radix: digit window, guard prefixes (below / above the window), digit
   // prefixes of 2^s keys holding nbd exact sub-digits each
   uint32_t glo = 0, ndp = 0, nbd = 1;
+  const bool refine = sd.mode == MODE_RADIX && (sd.flags & SEG_REFINE);  // uniform
+  bool hbins = hgram && bl == (int)W;  // the prefixes are bins of k_sample's histogram
   if (sd.mode == MODE_RADIX) {
     const uint32_t D = (uint32_t)bitlen<KT>(kmin ^ kmax);  // low bits the sampled keys differ in
     const uint32_t db = D < sd.radix_bits ? D : sd.radix_bits;
-    const uint32_t dpb = db < kMaxPrefixBits - 1 ? db : kMaxPrefixBits - 1;
+    // (a refined digit's prefix takes all of the LUT's bits where no key can
+    // lie beyond the window: its counts are then k_sample's histogram)
+    const uint32_t room = refine ? sd.pbits - (D < W ? 1u : 0u) : kMaxPrefixBits - 1;
+    const uint32_t dpb = db < room ? db : room;
     s = D - dpb;
     nbd = 1u << (db - dpb);
     ndp = 1u << dpb;
@@ -961,12 +968,13 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
     glo = base > 0 ? 1u : 0u;
     kb = (KT)(base - ((KT)glo << s));
     P = glo + ndp + (top < KeyBits<KT>::MAX ? 1u : 0u);
+    hbins = hgram && D >= W && dpb == sd.pbits;
     pb = (uint32_t)bitlen<uint32_t>(P - 1);
   } else if (sd.mode == MODE_RANGE) {
     pb = 0;
     s = (uint32_t)bl;
     P = 1;
-  } else if (hgram && bl == (int)W) {
+  } else if (hbins) {
     // full-width range with k_sample's histogram: prefixes aligned to
     // multiples of 2^s, so the prefix of a key is (key >> s) - (kb >> s)
     // and its count is hgram[key >> s]
@@ -993,7 +1001,7 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   uint32_t Btot, nsum = 0;
   bool spec = false;
 
-  if (sd.mode == MODE_RADIX) {
+  if (sd.mode == MODE_RADIX && !refine) {
     for (uint32_t p = tid; p < P; p += kThreads) {
       if (p < glo) lut[p] = 0u | (1u << 16);
       else if (p < glo + ndp) lut[p] = (glo + (p - glo) * nbd) | (nbd << 16);
@@ -1005,7 +1013,7 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
     if (tid == 0) lut[0] = nb << 16;
     Btot = nb;
   } else {
-    const bool useh = hgram && bl == (int)W;  // uniform
+    const bool useh = hbins;  // uniform
     if (useh && part != 0) return;  // uniform: one work-group reads the counts
     for (uint32_t p = tid; p < P; p += kThreads) reinterpret_cast<uint4*>(cnt4)[p] = make_uint4(0, 0, 0, 0);
     __syncthreads();
@@ -1154,7 +1162,7 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
   }
   // k_sample counts into a zeroed histogram: clear it for the next select
   // (every read of it is behind the barriers above)
-  if (hgram && sd.mode == MODE_SAMPLE)
+  if (hgram && seg_sampled(sd))
     for (uint32_t i = tid; i < (1u << sd.pbits); i += kThreads) hgram[i] = 0;
 }
 

@@ -172,12 +172,22 @@ inline uint64_t seg_heavy_max(uint64_t len, uint32_t nq) {
   return std::min<uint64_t>(nq, len / (kHeavyKeys + 1));
 }
 
+// Whether a radix segment's digits are refined (unless the second level is
+// switched off, where they stay plain).  A normal's keys crowd into a few
+// hundred of 2^14 digits: plain digits made the first compaction copy 88 % of
+// 2^27 floats for 1024 ranks and the second level read them twice more (809 us
+// a select); cut in proportion to the sample, 3 % is left (275 us, 14 of them
+// in the second level's three launches, which find nothing).  A fixed
+// digit width asked for (radix_bits) keeps its budget, the default takes the
+// sampled path's budget for the length.
+inline bool seg_refine(const ggks_opts& o, uint32_t mode) { return mode == MODE_RADIX && o.level2 >= 0; }
+
 // Whether a segment's active buckets are worth predicting: a sampled segment
 // whose ranks can lie in few places, long enough for the second pass over it
 // to cost more than the prediction, with chunks whose counts leave a histogram
 // word's top bit free.
-inline bool seg_spec(uint32_t mode, bool topk, uint64_t len, uint64_t chunk, uint32_t nq) {
-  return mode == MODE_SAMPLE && (topk || nq <= kSpecRanks) && len >= kSpecMinLen && chunk <= (1ull << 30);
+inline bool seg_spec(bool sampled, bool topk, uint64_t len, uint64_t chunk, uint32_t nq) {
+  return sampled && (topk || nq <= kSpecRanks) && len >= kSpecMinLen && chunk <= (1ull << 30);
 }
 
 // Second-level regions at the end of an arena layout (tables and scratch
@@ -201,6 +211,7 @@ inline void layout_level2(Plan& p, Take&& take, uint64_t red, uint64_t nq, int e
 struct SingleShape {
   bool direct;        // the whole vector fits the finisher's LDS
   uint32_t mode, rb;  // SegMode and radix digit width
+  bool refine;        // SEG_REFINE
   uint32_t bmax, pb;  // bucket budget, LUT prefix bits
   uint32_t ns;        // samples
   uint32_t nitems;    // reduce items
@@ -223,8 +234,13 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
     sh.mode = MODE_RADIX;
     uint32_t rb = o.radix_bits ? (uint32_t)o.radix_bits : 14u;
     sh.rb = std::min<uint32_t>(14, std::max<uint32_t>(4, rb));
+    sh.refine = seg_refine(o, sh.mode);
     bl = radix_budget_log2(sh.rb);
     sh.pb = radix_lut_bits(sh.rb);
+    if (sh.refine && !o.radix_bits) {
+      bl = t.buckets_log2;
+      sh.pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
+    }
   } else {
     bl = o.buckets_log2 ? (uint32_t)o.buckets_log2 : t.buckets_log2;
     bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
@@ -269,7 +285,8 @@ inline SegDesc single_segment(const SingleShape& sh, int kind, uint64_t n, uint3
   s.radix_bits = sh.rb;
   s.qsrc = kind == GGKS_KIND_TOPK ? QSRC_TOPK : QSRC_K;
   s.out_off = 0;
-  s.flags = seg_spec(sh.mode, kind == GGKS_KIND_TOPK, n, sh.csz, nq) ? SEG_SPEC : 0u;
+  s.flags = sh.refine ? SEG_REFINE : 0u;
+  if (seg_spec(sh.mode == MODE_SAMPLE || sh.refine, kind == GGKS_KIND_TOPK, n, sh.csz, nq)) s.flags |= SEG_SPEC;
   return s;
 }
 
@@ -346,8 +363,8 @@ inline void plan_single(Plan& p, int kind, int dtype, uint64_t n, uint32_t nq,
   p.nchunks = (uint32_t)G;
   p.nitems = sh.nitems;
   p.nsblocks = ns / kThreads;
-  p.lut_parts = ggks::lut_parts(sh.mode, ns, (uint32_t)eb);
-  p.emax_keys = sh.mode == MODE_RADIX ? n : (n + bmax - 1) / bmax;
+  p.lut_parts = ggks::lut_parts(sh.mode == MODE_SAMPLE || sh.refine, ns, (uint32_t)eb);
+  p.emax_keys = sh.mode == MODE_RADIX && !sh.refine ? n : (n + bmax - 1) / bmax;
 
   p.off_tables = off;
   p.off_segs = take(sizeof(SegDesc));
@@ -490,8 +507,11 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
       rb = std::min<uint32_t>(14, std::max<uint32_t>(4, rb));
       bl = radix_budget_log2(rb);
       pb = radix_lut_bits(rb);
-    } else {
-      bl = o.buckets_log2 ? (uint32_t)o.buckets_log2 : (bt.buckets_log2 ? bt.buckets_log2 : 12u);
+    }
+    const bool refine = seg_refine(o, mode);
+    if (mode == MODE_SAMPLE || (refine && !o.radix_bits)) {
+      bl = o.buckets_log2 && mode == MODE_SAMPLE ? (uint32_t)o.buckets_log2
+                                                 : (bt.buckets_log2 ? bt.buckets_log2 : 12u);
       bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
       pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
     }
@@ -540,7 +560,8 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     s.radix_bits = rb;
     s.qsrc = topk ? QSRC_TOPK : QSRC_K;
     s.out_off = (uint32_t)g.out_offset;
-    s.flags = seg_spec(mode, topk, n, csz, g.num_k) ? SEG_SPEC : 0u;
+    s.flags = refine ? SEG_REFINE : 0u;
+    if (seg_spec(mode == MODE_SAMPLE || refine, topk, n, csz, g.num_k)) s.flags |= SEG_SPEC;
     if (seg_level2(o, mode)) {
       const uint64_t hm = seg_heavy_max(n, g.num_k);
       if (hm > 0) {
@@ -588,12 +609,12 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
   // each: split builds would only add work-groups that exit at once
   if (p.segs.size() <= kLutSplitSegs)
     for (const SegDesc& sd : p.segs)
-      p.lut_parts = std::max(p.lut_parts, ggks::lut_parts(sd.mode, sd.nsample, (uint32_t)eb));
+      p.lut_parts = std::max(p.lut_parts, ggks::lut_parts(seg_sampled(sd), sd.nsample, (uint32_t)eb));
   p.ndirect = (uint32_t)p.direct_children.size();
   for (const Child& c : p.direct_children) p.dmax_keys = std::max<uint64_t>(p.dmax_keys, c.len);
   for (const SegDesc& sd : p.segs)
     p.emax_keys = std::max<uint64_t>(
-        p.emax_keys, sd.mode == MODE_RADIX ? sd.len : (sd.len + sd.bmax - 1) / sd.bmax);
+        p.emax_keys, !seg_sampled(sd) ? sd.len : (sd.len + sd.bmax - 1) / sd.bmax);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     size_t at = off;

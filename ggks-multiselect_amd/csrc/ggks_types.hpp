@@ -29,7 +29,7 @@ enum QuerySource : uint32_t {
 // Bucket-function modes of a segment.
 enum SegMode : uint32_t {
   MODE_SAMPLE = 0,  // prefix LUT sized from a random sample of the segment
-  MODE_RADIX = 1,   // the top radix_bits bits of the key (MSD radix digit)
+  MODE_RADIX = 1,   // the top radix_bits bits of the key (MSD radix digit), refined with SEG_REFINE
   MODE_RANGE = 2    // equal-width buckets over the known key range [lo, hi]
 };
 
@@ -64,7 +64,8 @@ struct SegDesc {          // planned on the host, read-only on the device
 
 enum SegFlags : uint32_t {
   SEG_LEVEL2 = 1u,
-  SEG_SPEC = 2u  // k_lut predicts its active buckets (Candidates, below)
+  SEG_SPEC = 2u,   // k_lut predicts its active buckets (Candidates, below)
+  SEG_REFINE = 4u  // MODE_RADIX: a digit's sub-digits in proportion to its share of the sample
 };
 
 // Candidates.  Where a segment's ranks lie in few places (a top-K, a cluster,
@@ -152,9 +153,15 @@ constexpr uint32_t kLutSplitBytes = 256u << 10;
 #if defined(__HIPCC__)
 __host__ __device__
 #endif
-inline uint32_t lut_parts(uint32_t mode, uint32_t nsample, uint32_t key_bytes) {
+inline bool seg_sampled(const SegDesc& sd) {  // its buckets follow the sample's shares
+  return sd.mode == MODE_SAMPLE || (sd.flags & SEG_REFINE);
+}
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline uint32_t lut_parts(bool sampled, uint32_t nsample, uint32_t key_bytes) {
   const uint64_t bytes = (uint64_t)nsample * key_bytes;
-  return (mode == MODE_SAMPLE && bytes > kLutSplitBytes) ? (uint32_t)(bytes / kLutPartBytes) : 1u;
+  return (sampled && bytes > kLutSplitBytes) ? (uint32_t)(bytes / kLutPartBytes) : 1u;
 }
 
 struct Chunk {            // one work-group of the streaming passes

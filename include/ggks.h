@@ -60,7 +60,8 @@ typedef struct ggks_opts {
   int32_t buckets_log2; /* bucket budget as log2 (8..15); 0 = tuned */
   int32_t destructive;  /* accepted; the input is never modified */
   uint64_t seed;        /* seed of the splitter sample; 0 = fixed default */
-  int32_t radix_bits;   /* radix path: digit width per level (4..14); 0 = 14 */
+  int32_t radix_bits;   /* radix path: digit width per level (4..14); 0 = 14
+                           (with a bucket budget tuned to the length) */
   int32_t level2;       /* second level for children of more than 2^16 keys
                            (re-bucketed by the whole GPU): 0 = radix plans
                            only, 1 = every plan, -1 = never */
@@ -101,7 +102,9 @@ int ggks_bucket_multiselect_i32(const int32_t *d_vec, int64_t n,
 
 /* Replaces RadixSelect::RadixSelectWrapper (merrillSelect.cu:210-259) and
  * InplaceRadix::inplaceRadixSelectWrapper (inplaceRadixSelect.cu:83-108),
- * generalised to many k: MSD digits of the converted key, no sampling. */
+ * generalised to many k: MSD digits of the converted key; a digit that holds
+ * a large share of a sample of the vector is cut into more sub-digits (plain
+ * digits with opts->level2 = -1). */
 int ggks_radix_multiselect(ggks_ctx *ctx, int dtype, const void *d_vec,
                            int64_t n, const uint32_t *h_k, int64_t num_k,
                            void *h_out, const ggks_opts *opt);
