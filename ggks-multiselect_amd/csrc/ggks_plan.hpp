@@ -239,6 +239,7 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
     sh.pb = radix_lut_bits(sh.rb);
     if (sh.refine && !o.radix_bits) {
       bl = t.buckets_log2;
+      sh.rb = std::min<uint32_t>(sh.rb, bl - 1);  // whole digits fit the budget
       sh.pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
     }
   } else {
@@ -514,6 +515,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
                                                  : (bt.buckets_log2 ? bt.buckets_log2 : 12u);
       bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
       pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
+      rb = std::min<uint32_t>(rb, bl - 1);
     }
     const uint32_t bmax = 1u << bl;
     uint64_t csz = 1ull << (bt.chunk_log2 ? bt.chunk_log2 : 16);
