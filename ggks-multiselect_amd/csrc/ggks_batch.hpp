@@ -192,6 +192,8 @@ static int batch_create(ggks_batch** out, int device, int dtype, const ggks_segm
   if (hipMemcpyAsync(b->arena + b->plan.off_tables, tab.data(), tb, hipMemcpyHostToDevice,
                      b->stream) != hipSuccess ||
       hipMemsetAsync(b->status, 0, 256, b->stream) != hipSuccess ||
+      (b->plan.small &&
+       hipMemsetAsync(b->arena + b->plan.off_tot, 0, (size_t)b->plan.ntot * 4, b->stream) != hipSuccess) ||
       hipStreamSynchronize(b->stream) != hipSuccess) {
     const hipError_t e = hipGetLastError();
     return bail(fail(GGKS_EDEVICE, "batch table upload failed: %s", hipGetErrorString(e)));
@@ -207,7 +209,11 @@ static int batch_run(ggks_batch* b, const void* d_vec, void* d_out, int flags) {
     return fail(GGKS_EINVAL, "null vector or output");
   std::lock_guard<std::mutex> lk(b->mu);
   HIP_TRY(hipSetDevice(b->device));
-  if (!(flags & GGKS_BATCH_GRAPH)) return batch_enqueue(b, d_vec, d_out);
+  if (!(flags & GGKS_BATCH_GRAPH)) {
+    const int rc = batch_enqueue(b, d_vec, d_out);
+    if (rc && b->plan.small) clear_words(b->stream, b->arena + b->plan.off_tot, b->plan.ntot);
+    return rc;
+  }
   if (b->exec && (b->g_src != d_vec || b->g_out != d_out)) batch_drop_graph(b);
   if (!b->exec) {
     HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));

@@ -758,6 +758,29 @@ constexpr uint64_t finish_small_reg_keys(bool lite) {
 // block's kThreads samples (3.1 %): it then gets a bucket of its own.
 constexpr uint32_t kHeavyMinCount = 32;
 
+// The state of a bucket function of P prefixes of 2^s keys from kb, Btot
+// buckets in all, without a heavy value.
+template <typename KT>
+__device__ __forceinline__ SegState lut_state(KT kb, KT kmax, uint32_t s, uint32_t P, uint32_t pb,
+                                              uint32_t Btot) {
+  SegState st = {};
+  st.kb = (uint64_t)kb;
+  st.kmax = (uint64_t)kmax;
+  // lmax = min(P * 2^s - 1, KMAX - kb): every key maps into a prefix < P
+  const unsigned __int128 span = ((unsigned __int128)P << s) - 1;
+  const unsigned __int128 room = (unsigned __int128)(KeyBits<KT>::MAX - kb);
+  st.lmax = (uint64_t)(span < room ? span : room);
+  st.s = s;
+  st.P = P;
+  st.B = Btot;
+  st.pwid = P > 1 ? pb : 0;
+  st.poff = P > 1 ? s : 0;
+  st.twid = s < 24 ? s : 24;
+  st.rsh = s > 24 ? s - 24 : 0;
+  st.lsh = s < 24 ? 24 - s : 0;
+  return st;
+}
+
 // Mark the buckets that can hold a segment's ranks.  A rank r of n has about
 // x = r S / n of the S samples below it, give or take the binomial deviation:
 // its bucket lies between those of sample positions x - d and x + d with
@@ -1130,25 +1153,7 @@ __global__ __launch_bounds__(kThreads) void k_lut(const SegDesc* __restrict__ se
     if (spec && tid < nmark) bits_pool[sd.bits_off + tid] = mark[tid];
   }
   if (tid == 0) {
-    SegState st = {};
-    st.kb = (uint64_t)kb;
-    st.kmax = (uint64_t)kmax;
-    // lmax = min(P * 2^s - 1, KMAX - kb): every key maps into a prefix < P
-    const unsigned __int128 span = ((unsigned __int128)P << s) - 1;
-    const unsigned __int128 room = (unsigned __int128)(KeyBits<KT>::MAX - kb);
-    st.lmax = (uint64_t)(span < room ? span : room);
-    st.s = s;
-    st.P = P;
-    st.B = Btot;
-    st.nact = 0;
-    st.pwid = P > 1 ? pb : 0;
-    st.poff = P > 1 ? s : 0;
-    st.twid = s < 24 ? s : 24;
-    st.rsh = s > 24 ? s - 24 : 0;
-    st.lsh = s < 24 ? 24 - s : 0;
-    st.hvon = 0;
-    st.hv = 0;
-    st.hb = 0;
+    SegState st = lut_state<KT>(kb, kmax, s, P, pb, Btot);
     st.arrive = spec ? 1u : 0u;
     if (hvon) {  // hv's bucket is L(hv) + 1; two more buckets in all
       BucketFn<KT> fn;
@@ -1488,8 +1493,9 @@ __device__ __forceinline__ uint32_t seg_out(const SegDesc& sd, const Query* __re
 // of bucket prefixes a thread holds: the full instance takes up to
 // kMaxBuckets buckets, the small one up to 4096 in at most 64 VGPRs, so that
 // two work-groups share a CU (batches of many segments).
-template <typename KT, int C, uint32_t TV>
-__device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
+// RAW: the totals are plain counts (k_front's), not k_reduce's prefixes.
+template <typename KT, int C, uint32_t TV, bool RAW>
+__device__ __forceinline__ void findk_segment(uint32_t sg, const SegDesc* __restrict__ segs,
                                               SegState* __restrict__ states,
                                               const uint32_t* __restrict__ lut_pool,
                                               const uint32_t* __restrict__ totals,
@@ -1510,7 +1516,7 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
                                               uint32_t* __restrict__ bigw,
                                               uint2* __restrict__ cinfo) {
   extern __shared__ __align__(16) uint32_t lds[];
-  const SegDesc sd = segs[blockIdx.x];
+  const SegDesc sd = segs[sg];
   // the first k of this thread, read now so its latency hides under the
   // table loads and scans
   const uint32_t kfirst =
@@ -1536,28 +1542,38 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
   for (uint32_t u = 0; u < TV; ++u)
     if (tid + u * kThreads < nt4) tv[u] = tot4[tid + u * kThreads];
   uint4 gv = make_uint4(0, 0, 0, 0), lv = make_uint4(0, 0, 0, 0);
-  if (tid < ng4) gv = reinterpret_cast<const uint4*>(gsums + sd.tot_off / kReduceBins)[tid];
+  if (!RAW && tid < ng4) gv = reinterpret_cast<const uint4*>(gsums + sd.tot_off / kReduceBins)[tid];
   if (tid < nl4) lv = reinterpret_cast<const uint4*>(lut_pool + sd.lut_off)[tid];
   // a candidate word of k_lut's (kSpecShare), where it left any
   const uint32_t cw =
       (sd.flags & SEG_SPEC) && tid < wcap ? bits_pool[sd.bits_off + tid] : 0u;
   __shared__ SegState st;
-  if (threadIdx.x == 0) st = states[blockIdx.x];
-  if (tid < ng4) reinterpret_cast<uint4*>(wc)[tid] = gv;
+  if (threadIdx.x == 0) st = states[sg];
+  if (!RAW && tid < ng4) reinterpret_cast<uint4*>(wc)[tid] = gv;
   if (tid < nl4) reinterpret_cast<uint4*>(lut)[tid] = lv;
   __syncthreads();
   const uint32_t B = st.B;
   const uint32_t nwords = (B + 31) / 32;
   const uint32_t ngroups = (B + kReduceBins - 1) / kReduceBins;  // <= wcap
   for (uint32_t i = tid; i < nwords; i += kThreads) bits[i] = 0;
-  const uint32_t len = block_scan_array(wc, ngroups, wsum);  // group bases (synchronises)
+  uint32_t len;
+  if constexpr (RAW) {
+    static_assert(TV == 1, "one word of counts a thread");
+    if (tid >= nt4) tv[0] = make_uint4(0, 0, 0, 0);
+    const uint4 t = tv[0];
+    const uint32_t e = block_excl_scan(t.x + t.y + t.z + t.w, wsum, len);
+    if (tid < nt4)
+      reinterpret_cast<uint4*>(hist)[tid] = make_uint4(e, e + t.x, e + t.x + t.y, e + t.x + t.y + t.z);
+  } else {
+    len = block_scan_array(wc, ngroups, wsum);  // group bases (synchronises)
 #pragma unroll
-  for (uint32_t u = 0; u < TV; ++u) {
-    const uint32_t i4 = tid + u * kThreads;
-    if (i4 < nt4) {
-      const uint32_t g = wc[i4 * 4 / kReduceBins];
-      reinterpret_cast<uint4*>(hist)[i4] =
-          make_uint4(tv[u].x + g, tv[u].y + g, tv[u].z + g, tv[u].w + g);
+    for (uint32_t u = 0; u < TV; ++u) {
+      const uint32_t i4 = tid + u * kThreads;
+      if (i4 < nt4) {
+        const uint32_t g = wc[i4 * 4 / kReduceBins];
+        reinterpret_cast<uint4*>(hist)[i4] =
+            make_uint4(tv[u].x + g, tv[u].y + g, tv[u].z + g, tv[u].w + g);
+      }
     }
   }
   __syncthreads();  // hist = exclusive prefix of the bucket counts
@@ -1645,7 +1661,7 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
     c.q_cnt = 0;
     c.src = 1;
     c.bucket = b;
-    c.seg = blockIdx.x;
+    c.seg = sg;
     children[sd.q_off + u] = c;
     cinfo[sd.q_off + u] = make_uint2(start, b);
   }
@@ -1729,7 +1745,7 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
         H.len = clen;
         H.lo = cp->lo;
         H.hi = cp->hi;
-        H.seg = blockIdx.x;
+        H.seg = sg;
         H.slot = sd.q_off + u;
         H.q_off = sd.q_off + first;
         H.q_cnt = next - first;
@@ -1755,7 +1771,7 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
     }
     if (big_child(cp->len, cp->q_cnt)) atomicAdd(&lbig, 1u);
   }
-  if (l2 && tid == 0) states[blockIdx.x].nfree = U;  // first free child slot
+  if (l2 && tid == 0) states[sg].nfree = U;  // first free child slot
   __syncthreads();
   for (uint32_t i = tid; i < sd.q_cnt; i += kThreads) {
     uint32_t u = qb[sd.q_off + i];
@@ -1773,11 +1789,11 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
     children[sd.q_off + u].len = 0;
   }
   if (tid == 0) {
-    states[blockIdx.x].nact = U;
-    states[blockIdx.x].nred = mtot;
+    states[sg].nact = U;
+    states[sg].nred = mtot;
     // the compaction reads the candidates: all there, and its children end
     // below them
-    states[blockIdx.x].arrive = st.arrive && !miss && mtot <= spec_area(sd.len, 0) ? 1u : 0u;
+    states[sg].arrive = st.arrive && !miss && mtot <= spec_area(sd.len, 0) ? 1u : 0u;
     if (bigw && lbig) atomicAdd(bigw, lbig);
   }
 }
@@ -1797,15 +1813,370 @@ __device__ __forceinline__ void findk_segment(const SegDesc* __restrict__ segs,
 constexpr uint32_t kFindkSmallBuckets = 4 * kThreads;  // one 16-byte word per thread
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) void k_findk(GGKS_FINDK_PARAMS) {
-  findk_segment<KT, C, kMaxBuckets / 4 / kThreads>(GGKS_FINDK_ARGS);
+  findk_segment<KT, C, kMaxBuckets / 4 / kThreads, false>(blockIdx.x, GGKS_FINDK_ARGS);
 }
 template <typename KT, int C>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_findk_small(
     GGKS_FINDK_PARAMS) {
-  findk_segment<KT, C, 1>(GGKS_FINDK_ARGS);
+  findk_segment<KT, C, 1, false>(blockIdx.x, GGKS_FINDK_ARGS);
+}
+
+// ------------------------------------------------------- short segments
+// Plans whose segments are all short (less than 16 MiB of keys, at most 4096
+// buckets and 1024 ranks; Plan::small) run two kernels in place of k_sample,
+// k_lut, k_count, k_reduce, k_findk and k_compact.  Such selects are bound by
+// launches and by each kernel's chain of dependent round trips, not by
+// bandwidth, so work-groups repeat what used to be handed from one kernel to
+// the next: every chunk's work-group samples the segment and builds its
+// bucket function (k_front), and scans the bucket totals and finds the active
+// buckets (k_back).  A chunk is what a work-group holds in registers, so
+// each pass is one round of loads, and the chunks' counts meet in device-scope
+// atomics instead of rows.  2^20 floats, 101 ranks: six kernels of 39 us in
+// all before, two of 22 us (a synchronous call 78.6 -> 56.6 us).
+constexpr int kSmallWords = 4;  // 16-byte words of a chunk per thread
+template <typename KT>
+constexpr uint32_t kSmallChunk = kSmallWords * kThreads * 16 / sizeof(KT);
+constexpr uint32_t kSmallBuckets = 4096, kSmallPrefixes = 2048, kSmallRanks = 1024, kSmallSamples = 4096;
+
+// A chunk's keys: 16-byte words in registers, at most one unaligned head and
+// one tail key a thread.
+template <typename KT>
+struct ChunkKeys {
+  static constexpr uint32_t VEC = 16 / sizeof(KT);
+  static constexpr int N = kSmallWords * (int)VEC;
+  uint4 v[kSmallWords];
+  KT hk, tk;
+  uint32_t nv;  // words of this thread
+  bool hh, ht;
+  __device__ __forceinline__ void load(const KT* __restrict__ p, uint32_t len) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t mis = (uint32_t)((uintptr_t)p & 15u) / sizeof(KT);
+    uint32_t head = mis ? VEC - mis : 0u;
+    if (head > len) head = len;
+    const uint32_t nvec = (len - head) / VEC;  // <= kSmallWords * kThreads
+    const uint4* __restrict__ pv = reinterpret_cast<const uint4*>(p + head);
+    nv = nvec > tid ? (nvec - tid + kThreads - 1) / kThreads : 0u;
+#pragma unroll
+    for (int u = 0; u < kSmallWords; ++u)
+      v[u] = (uint32_t)u < nv ? pv[tid + u * kThreads] : make_uint4(0, 0, 0, 0);
+    hh = tid < head;
+    hk = hh ? p[tid] : KT(0);
+    const uint32_t done = head + nvec * VEC;
+    ht = done + tid < len;
+    tk = ht ? p[done + tid] : KT(0);
+  }
+};
+
+// Sample, bucket function and count.  Grid: the chunks, and one more
+// work-group that copies the call's k list from pinned host memory.
+template <typename KT, int C>
+__global__ __launch_bounds__(kThreads) void k_front(const KT* __restrict__ src,
+                                                    const SegDesc* __restrict__ segs,
+                                                    const Chunk* __restrict__ chunks, uint32_t nchunks,
+                                                    uint64_t seed, SegState* __restrict__ states,
+                                                    uint32_t* __restrict__ lut_pool,
+                                                    uint32_t* __restrict__ totals,
+                                                    uint32_t* __restrict__ cursors,
+                                                    uint32_t* __restrict__ bigw,
+                                                    const uint32_t* __restrict__ hk,
+                                                    uint32_t* __restrict__ dk, uint32_t nk) {
+  __shared__ uint32_t hist[kSmallBuckets];
+  __shared__ uint32_t lut[kSmallPrefixes], cnt[kSmallPrefixes];
+  __shared__ KT red_lo[16], red_hi[16], cand[16];
+  __shared__ uint32_t ccnt[16][16], wsum[17];
+  __shared__ KT sh_lo, sh_hi, sh_hv;
+  __shared__ uint32_t sh_hvon;
+  __shared__ SegState st;
+  constexpr uint32_t W = KeyBits<KT>::W, NS = kSmallSamples / kThreads;
+  const uint32_t tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+  if (blockIdx.x >= nchunks) {
+    for (uint32_t i = tid; i < nk; i += kThreads) dk[i] = hk[i];
+    return;
+  }
+  const Chunk ch = chunks[blockIdx.x];
+  const SegDesc sd = segs[ch.seg];
+  ChunkKeys<KT> ck;
+  // the sample's gathers first: they are waited for first
+  KT k[NS];
+#pragma unroll
+  for (uint32_t j = 0; j < NS; ++j) {
+    const uint32_t i = j * kThreads + tid;
+    uint64_t z = seed + 0x9E3779B97F4A7C15ull * ((uint64_t)ch.seg * 0x100000001ull + i + 1);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    k[j] = i < sd.nsample ? src[sd.data_off + __umul64hi(z, sd.len)] : KT(0);
+  }
+  ck.load(src + sd.data_off + ch.start, (uint32_t)ch.len);
+  for (uint32_t i = tid; i < kSmallBuckets; i += kThreads) hist[i] = 0;
+  for (uint32_t i = tid; i < kSmallPrefixes; i += kThreads) cnt[i] = 0;
+  KT lo = KeyBits<KT>::MAX, hi = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < NS; ++j) {
+    if (j * kThreads < sd.nsample) {  // uniform (sample counts are multiples of 1024)
+      k[j] = to_key<C>(k[j]);
+      lo = k[j] < lo ? k[j] : lo;
+      hi = k[j] > hi ? k[j] : hi;
+    }
+  }
+  if (lane == 0) cand[w] = k[0];
+  for (int d = 32; d >= 1; d >>= 1) {
+    const KT a = __shfl_xor(lo, d, 64), b = __shfl_xor(hi, d, 64);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  if (lane == 0) {
+    red_lo[w] = lo;
+    red_hi[w] = hi;
+  }
+  __syncthreads();  // cand, red_lo / red_hi, cleared tables
+  // copies of every wavefront's proposal (k_sample's heavy value)
+#pragma unroll
+  for (uint32_t c = 0; c < 16; ++c) {
+    const KT cv = cand[c];
+    uint32_t m = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < NS; ++j)
+      if (j * kThreads < sd.nsample) m += (uint32_t)__popcll(__ballot(k[j] == cv));
+    if (lane == 0) ccnt[w][c] = m;
+  }
+  __syncthreads();
+  if (w == 0) {
+    uint32_t t = 0;
+    KT cv = KeyBits<KT>::MAX, l = KeyBits<KT>::MAX, h = 0;
+    if (lane < 16) {
+      for (uint32_t v = 0; v < 16; ++v) t += ccnt[v][lane];
+      cv = cand[lane];
+      l = red_lo[lane];
+      h = red_hi[lane];
+    }
+    for (int d = 8; d >= 1; d >>= 1) {
+      const KT la = __shfl_xor(l, d, 64), ha = __shfl_xor(h, d, 64);
+      l = la < l ? la : l;
+      h = ha > h ? ha : h;
+      const uint32_t ot = (uint32_t)__shfl_xor((int)t, d, 64);
+      const KT oc = __shfl_xor(cv, d, 64);
+      if (ot > t || (ot == t && oc < cv)) {
+        t = ot;
+        cv = oc;
+      }
+    }
+    if (lane == 0) {
+      sh_lo = l;
+      sh_hi = h;
+      sh_hv = cv;
+      sh_hvon = t * kThreads >= kHeavyMinCount * sd.nsample ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+  const KT kmin = sh_lo, kmax = sh_hi;
+  const uint32_t hvon = sh_hvon;
+  // k_lut's prefixes over the sampled range, guards where there is room
+  const KT R = kmax - kmin;
+  const int bl = bitlen<KT>(R);
+  const uint32_t pb = sd.pbits;
+  const uint32_t s = bl > (int)pb ? (uint32_t)(bl - (int)pb) : 0u;
+  uint32_t P = (uint32_t)(((uint64_t)R >> s) + 1);
+  KT kb = kmin;
+  if (P + 2 <= (1u << pb)) {
+    const uint32_t glo = kmin >= (KT(1) << s) ? 1u : 0u;
+    kb = (KT)(kmin - ((KT)glo << s));
+    const bool ghi = (KT)(KeyBits<KT>::MAX - kb) >> s >= (KT)(P + glo);
+    P += glo + (ghi ? 1u : 0u);
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < NS; ++j)
+    if (j * kThreads < sd.nsample) atomicAdd(&cnt[(uint32_t)((KT)(k[j] - kb) >> s)], 1u);
+  __syncthreads();
+  const uint32_t Bt = sd.bmax - (hvon ? 2u : 0u);
+  const uint32_t cap = s >= 16 ? 65535u : min(65535u, 1u << s);
+  constexpr uint32_t PT = kSmallPrefixes / kThreads;  // prefixes per thread
+  uint32_t c[PT], nonempty = 0, runs = 0;
+  const uint32_t cprev = tid > 0 ? cnt[tid * PT - 1] : 1u;
+#pragma unroll
+  for (uint32_t u = 0; u < PT; ++u) {
+    const uint32_t p = tid * PT + u;
+    c[u] = p < P ? cnt[p] : 0u;
+    if (p < P) {
+      if (c[u]) nonempty++;
+      else if (p == 0 || (u > 0 ? c[u > 0 ? u - 1 : 0] : cprev)) runs++;
+    }
+  }
+  uint32_t t12;
+  block_excl_scan(nonempty | (runs << 16), wsum, t12);
+  const uint32_t used = (t12 & 0xFFFFu) + (t12 >> 16);
+  const uint32_t A = Bt > used ? Bt - used : 0u;
+  uint32_t nb[PT], wd[PT], local = 0;
+#pragma unroll
+  for (uint32_t u = 0; u < PT; ++u) {
+    const uint32_t p = tid * PT + u;
+    nb[u] = c[u] ? min(cap, 1u + c[u] * A / sd.nsample) : 0u;  // c A < 2^25
+    wd[u] = c[u] ? nb[u] : p < P && (p == 0 || (u > 0 ? c[u > 0 ? u - 1 : 0] : cprev)) ? 1u : 0u;
+    local += wd[u];
+  }
+  uint32_t Btot;
+  uint32_t run = block_excl_scan(local, wsum, Btot);
+#pragma unroll
+  for (uint32_t u = 0; u < PT; ++u) {
+    const uint32_t p = tid * PT + u;
+    if (p < P) lut[p] = (wd[u] == 0 ? run - 1 : run) | (nb[u] << 16);
+    run += wd[u];
+  }
+  __syncthreads();  // the LUT
+  if (tid == 0) {
+    SegState t = lut_state<KT>(kb, kmax, s, P, pb, Btot);
+    if (hvon) {
+      BucketFn<KT> fn;
+      fn.init(t);
+      t.hvon = 1;
+      t.hv = (uint64_t)sh_hv;
+      t.hb = fn(sh_hv, lut) + 1;
+      t.B = Btot + 2;
+    }
+    st = t;
+  }
+  __syncthreads();
+  BucketFn<KT> bk;
+  bk.init(st);
+  {
+    KT key[ChunkKeys<KT>::N];
+    unpack<KT, kSmallWords>(ck.v, key);
+    uint32_t b[ChunkKeys<KT>::N];
+    bucket_batch<KT, C, ChunkKeys<KT>::N>(bk, lut, key, b);
+#pragma unroll
+    for (int i = 0; i < ChunkKeys<KT>::N; ++i)
+      if ((uint32_t)i / ChunkKeys<KT>::VEC < ck.nv) lds_inc(hist, b[i]);
+    if (ck.hh) atomicAdd(&hist[bk(to_key<C>(ck.hk), lut)], 1u);
+    if (ck.ht) atomicAdd(&hist[bk(to_key<C>(ck.tk), lut)], 1u);
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < st.B; i += kThreads)
+    if (hist[i]) atomicAdd(&totals[sd.tot_off + i], hist[i]);
+  if (ch.idx == 0) {  // what k_back reads
+    for (uint32_t i = tid; i < P; i += kThreads) lut_pool[sd.lut_off + i] = lut[i];
+    for (uint32_t i = tid; i < sd.q_cnt; i += kThreads) cursors[sd.q_off + i] = 0;
+    if (tid == 0) {
+      states[ch.seg] = st;
+      if (ch.seg == 0) *bigw = 0;
+    }
+  }
+}
+
+// Ranks to buckets and compaction.  Grid: the chunks, whose work-groups each
+// find the active buckets, place their chunk's keys of them in LDS order and
+// take their places in the children by one atomic per child; and a work-group
+// per segment beside them, which writes the children and their ranks
+// (findk_segment).
+template <typename KT, int C>
+__global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
+                                                   const Chunk* __restrict__ chunks, uint32_t nchunks,
+                                                   uint32_t* __restrict__ cursors, KT* __restrict__ red,
+                                                   GGKS_FINDK_PARAMS) {
+  if (blockIdx.x >= nchunks) {
+    findk_segment<KT, C, 1, true>(blockIdx.x - nchunks, GGKS_FINDK_ARGS);
+    return;
+  }
+  extern __shared__ __align__(16) uint32_t lds[];
+  uint32_t* pre = lds;                      // bucket prefixes
+  uint32_t* lut = pre + kSmallBuckets;      // kSmallPrefixes
+  uint32_t* bits = lut + kSmallPrefixes;    // active buckets
+  uint32_t* wb = bits + kSmallBuckets / 32; // first child of a word
+  uint32_t* cstart = wb + kSmallBuckets / 32;  // per child: first place, then this chunk's
+  uint32_t* lcnt = cstart + kSmallRanks;       // per child: this chunk's keys
+  uint32_t* wsum = lcnt + kSmallRanks;         // 17
+  const uint32_t tid = threadIdx.x;
+  const Chunk ch = chunks[blockIdx.x];
+  const SegDesc sd = segs[ch.seg];
+  const uint32_t nt4 = sd.bmax / 4;
+  const uint4 t = tid < nt4 ? reinterpret_cast<const uint4*>(totals + sd.tot_off)[tid] : make_uint4(0, 0, 0, 0);
+  const uint32_t kfirst = sd.qsrc == QSRC_K && tid < sd.q_cnt ? kraw[sd.q_off + tid] : 0u;
+  const SegState st = states[ch.seg];  // (findk_segment writes other fields of it)
+  ChunkKeys<KT> ck;
+  ck.load(src + sd.data_off + ch.start, (uint32_t)ch.len);
+  for (uint32_t i = tid; i < st.P; i += kThreads) lut[i] = lut_pool[sd.lut_off + i];
+  if (tid < kSmallBuckets / 32) bits[tid] = 0;
+  lcnt[tid] = 0;
+  const uint32_t B = st.B;
+  uint32_t len;
+  const uint32_t e = block_excl_scan(t.x + t.y + t.z + t.w, wsum, len);
+  if (tid < nt4)
+    reinterpret_cast<uint4*>(pre)[tid] = make_uint4(e, e + t.x, e + t.x + t.y, e + t.x + t.y + t.z);
+  __syncthreads();
+  auto count_of = [&](uint32_t b) { return (b + 1 < B ? pre[b + 1] : len) - pre[b]; };
+  RangeOf<KT> range;
+  range.fn.init(st);
+  range.lut = lut;
+  range.B = B;
+  range.P = st.P;
+  range.s = st.s;
+  range.hb = st.hb;
+  // the active buckets, by findk_segment's rules (no more ranks than threads)
+  if (tid < sd.q_cnt) {
+    uint64_t kk = kfirst < 1 || (uint64_t)kfirst > sd.len ? 1 : kfirst;
+    const uint32_t r1 = (uint32_t)(sd.qsrc == QSRC_K ? sd.len - kk : sd.len - tid - 1);
+    uint32_t lo = 0, hi = B - 1;  // largest b with pre[b] <= r1
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi + 1) >> 1;
+      if (pre[mid] <= r1) lo = mid; else hi = mid - 1;
+    }
+    KT klo = 0, khi = 1;
+    if (st.s < 17 || (st.hvon && lo == st.hb)) range(lo, klo, khi);
+    if (klo != khi) lds_or(bits, lo >> 5, 1u << (lo & 31));
+  }
+  __syncthreads();
+  const uint32_t nwords = (B + 31) / 32;
+  uint32_t m = 0, csum = 0;
+  if (tid < nwords) {
+    m = bits[tid];
+    for (uint32_t mm = m; mm; mm &= mm - 1) csum += count_of(tid * 32 + __ffs(mm) - 1);
+  }
+  uint32_t U, mtot;
+  uint32_t u0 = block_excl_scan((uint32_t)__popc(m), wsum, U);
+  uint32_t c0 = block_excl_scan(csum, wsum, mtot);
+  if (tid < nwords) {
+    wb[tid] = u0;
+    for (uint32_t mm = m; mm; mm &= mm - 1) {
+      cstart[u0++] = c0;
+      c0 += count_of(tid * 32 + __ffs(mm) - 1);
+    }
+  }
+  __syncthreads();
+  if (U == 0) return;  // uniform
+  constexpr int N = ChunkKeys<KT>::N;
+  constexpr uint32_t NONE = 0xFFFFFFFFu;
+  KT key[N];
+  unpack<KT, kSmallWords>(ck.v, key);
+  uint32_t b[N];
+  bucket_batch<KT, C, N>(range.fn, lut, key, b);
+  // b: (child << 16) | place among this chunk's keys of the child, or NONE
+  auto take = [&](uint32_t bk, bool ok) {
+    const uint32_t wd = bits[bk >> 5], sh = bk & 31u;
+    if (!ok || !((wd >> sh) & 1u)) return NONE;
+    const uint32_t u = wb[bk >> 5] + __popc(wd & ((1u << sh) - 1u));
+    return (u << 16) | lds_inc(lcnt, u);
+  };
+#pragma unroll
+  for (int i = 0; i < N; ++i) b[i] = take(b[i], (uint32_t)i / ChunkKeys<KT>::VEC < ck.nv);
+  const uint32_t bh = take(range.fn(to_key<C>(ck.hk), lut), ck.hh);
+  const uint32_t bt = take(range.fn(to_key<C>(ck.tk), lut), ck.ht);
+  __syncthreads();
+  if (tid < U && lcnt[tid]) cstart[tid] += atomicAdd(&cursors[sd.q_off + tid], lcnt[tid]);
+  __syncthreads();
+  KT* const rseg = red + sd.red_base;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (b[i] != NONE) rseg[cstart[b[i] >> 16] + (b[i] & 0xFFFFu)] = key[i];
+  if (bh != NONE) rseg[cstart[bh >> 16] + (bh & 0xFFFFu)] = ck.hk;
+  if (bt != NONE) rseg[cstart[bt >> 16] + (bt & 0xFFFFu)] = ck.tk;
 }
 #undef GGKS_FINDK_PARAMS
 #undef GGKS_FINDK_ARGS
+
+// Clear n words (a kernel, so that a caller may capture it).
+__global__ __launch_bounds__(256) void k_clear(uint32_t* __restrict__ p, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
 
 // Pass 2 (k_compact): stream the chunk once and move the keys of active
 // buckets into their children's ranges (each chunk owns a private slice of
@@ -3306,7 +3677,10 @@ __global__ __launch_bounds__(kThreads) void k_finish(const KT* __restrict__ inpu
                                                      const Query* __restrict__ cq0,
                                                      const Query* __restrict__ cq2,
                                                      KT* __restrict__ out,
-                                                     const uint32_t* __restrict__ bigw) {
+                                                     const uint32_t* __restrict__ bigw,
+                                                     uint32_t* __restrict__ zero, uint32_t nzero) {
+  // k_front's totals, clear for the next select
+  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < nzero; i += gridDim.x * kThreads) zero[i] = 0;
   // nothing to do when k_findk counted no child for this finisher
   if (bigw && *bigw == 0) return;  // uniform
   constexpr uint32_t CAP = kFinishLdsBytes / sizeof(KT), S = CAP / kThreads;

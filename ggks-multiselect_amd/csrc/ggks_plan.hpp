@@ -105,12 +105,46 @@ inline uint32_t radix_lut_bits(uint32_t rb) { return std::min<uint32_t>(kMaxPref
 // Batches of at most this many segments split large segments' LUT builds.
 constexpr size_t kLutSplitSegs = 16;
 
+// Plans of short segments (k_front / k_back): less than 16 MiB of keys, at
+// most 12 bucket bits, 1024 ranks and 4096 samples each, 512 chunks in all.
+// A stream of selects of 1 / 100 / 1000 ranks, six kernels against two:
+// 65537 floats 44 / 47 / 55 -> 27 / 28 / 35 us, 2^20 doubles 51 / 54 / 73 ->
+// 30 / 34 / 40, 3e6 ints 50 / 51 / 63 -> 33 / 42 / 52; where every chunk's
+// work-group's own sample and scans come near what they save, at 4.1e6
+// doubles 68 / 72 / 127 -> 51 / 59 / 71 and 4.1e6 ints 53 / 55 / 72 ->
+// 39 / 48 / 59, the longer pipeline's candidates and wider tables start.
+constexpr uint64_t kSmallBytes = 1ull << 24;
+constexpr uint32_t kSmallBucketBits = 12, kSmallMaxRanks = 1024;
+constexpr uint64_t kSmallMaxChunks = 512;
+inline bool small_len(uint64_t n, int eb) { return n * (uint32_t)eb < kSmallBytes; }
+inline uint64_t small_chunk_keys(int eb) { return 4ull * kThreads * 16 / (uint32_t)eb; }
+// Chunk length of a short segment: 64 chunks of it (128: 1.2 us more at 5e5
+// keys), between 4096 keys and what a work-group holds.
+inline uint64_t small_chunk(uint64_t n, int eb) {
+  const uint64_t c = std::min<uint64_t>(small_chunk_keys(eb), std::max<uint64_t>(4096, n / 64));
+  return (c + 63) / 64 * 64;
+}
+// Every chunk's work-group draws the sample: 0.6 us per 1024 gathers.  2048
+// are enough (1024 to 2^17 keys), except where many ranks meet children that
+// leave the 256-thread finisher's registers (1000 ranks of 2^20 ints: 41.6 us
+// with 4096 samples, 51.5 with 2048; of 2^20 doubles: 43.4 and 40.4).
+inline uint32_t small_samples(uint64_t n, uint32_t nq, int eb) {
+  if (n <= 1ull << 17) return 1024;
+  return eb == 4 && nq > 128 && n > 1ull << 19 ? 4096 : 2048;
+}
+// LUT prefix bits: half the buckets, as the prefixes that hold a sample and the
+// runs between them take a bucket each at least.
+inline uint32_t small_lut_bits(uint32_t bl) { return bl - 1; }
+
 struct Plan {
   std::vector<SegDesc> segs;
   std::vector<Chunk> chunks;
   std::vector<ReduceItem> items;
   std::vector<Child> direct_children;
   bool direct = false;  // single-vector plan answered by the finisher alone
+  bool small = false;   // every engine segment is short (k_front / k_back)
+  size_t off_curs = 0;  // their children's cursors
+  uint32_t ntot = 0;    // their bucket totals, zero between runs
   uint32_t nq = 0;
   uint32_t qmax = 0;  // most ranks of one engine segment
   uint32_t bmax_max = 0;
@@ -146,7 +180,7 @@ struct Plan {
     if (!segs.empty()) memcpy(dst + (off_segs - off_tables), segs.data(), segs.size() * sizeof(SegDesc));
     if (!chunks.empty())
       memcpy(dst + (off_chunks - off_tables), chunks.data(), chunks.size() * sizeof(Chunk));
-    if (!items.empty())
+    if (!items.empty() && !small)  // (short segments have no reduce pass)
       memcpy(dst + (off_items - off_tables), items.data(), items.size() * sizeof(ReduceItem));
     if (!sblocks.empty())
       memcpy(dst + (off_sblocks - off_tables), sblocks.data(), sblocks.size() * sizeof(SampleBlock));
@@ -206,12 +240,35 @@ inline void layout_level2(Plan& p, Take&& take, uint64_t red, uint64_t nq, int e
   p.off_red2 = take((size_t)red * eb);
 }
 
+// The scratch of a plan of short segments (no sample, rows, group sums).  The
+// totals come last, so that they and a status block behind the plan are
+// cleared together.
+template <typename Take>
+inline void layout_small(Plan& p, Take&& take, size_t nseg, uint64_t luts, uint64_t tots, uint64_t bitw,
+                         uint64_t nq, uint64_t red, int eb) {
+  p.off_states = take(nseg * sizeof(SegState));
+  p.off_lut = take((size_t)luts * 4);
+  p.off_bits = take((size_t)bitw * 4);
+  p.off_wbase = take((size_t)bitw * 4);
+  p.off_qb = take((size_t)nq * 4);
+  p.off_qr = take((size_t)nq * 4);
+  p.off_children = take((size_t)nq * sizeof(Child));
+  p.off_cinfo = take((size_t)nq * 8);
+  p.off_cq = take((size_t)nq * sizeof(Query));
+  p.off_curs = take((size_t)nq * 4);
+  p.off_red = take((size_t)red * eb);
+  p.off_big = take(4);
+  p.ntot = (uint32_t)tots;
+  p.off_tot = take((size_t)tots * 4);
+}
+
 // The shape of a single-vector plan: its route, bucket function parameters,
 // chunking and sample size, computed from scalars alone (no tables).
 struct SingleShape {
   bool direct;        // the whole vector fits the finisher's LDS
   uint32_t mode, rb;  // SegMode and radix digit width
   bool refine;        // SEG_REFINE
+  bool small;         // k_front / k_back
   uint32_t bmax, pb;  // bucket budget, LUT prefix bits
   uint32_t ns;        // samples
   uint32_t nitems;    // reduce items
@@ -253,11 +310,18 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
   G = std::min<uint64_t>(G, kMaxChunks);
   uint64_t csz = (n + G - 1) / G;
   csz = (csz + 63) / 64 * 64;
+  sh.small = sh.mode == MODE_SAMPLE && o.level2 <= 0 && o.blocks <= 0 && small_len(n, eb) &&
+             bl <= kSmallBucketBits && nq <= kSmallMaxRanks;
+  if (sh.small) {
+    csz = small_chunk(n, eb);
+    sh.pb = small_lut_bits(bl);
+  }
   sh.G = (n + csz - 1) / csz;
   sh.csz = csz;
   {  // both modes sample: the LUT (bucket) or the digit window (radix)
     uint64_t want = (n / 256 + 1023) / 1024 * 1024;
-    sh.ns = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(4096, want));
+    sh.ns = sh.small ? small_samples(n, nq, eb)
+                     : (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(4096, want));
   }
   sh.gl = reduce_groups_log2(sh.G);
   const uint32_t ng = (sh.bmax + kReduceBins - 1) / kReduceBins;
@@ -287,7 +351,7 @@ inline SegDesc single_segment(const SingleShape& sh, int kind, uint64_t n, uint3
   s.qsrc = kind == GGKS_KIND_TOPK ? QSRC_TOPK : QSRC_K;
   s.out_off = 0;
   s.flags = sh.refine ? SEG_REFINE : 0u;
-  if (seg_spec(sh.mode == MODE_SAMPLE || sh.refine, kind == GGKS_KIND_TOPK, n, sh.csz, nq)) s.flags |= SEG_SPEC;
+  if (!sh.small && seg_spec(sh.mode == MODE_SAMPLE || sh.refine, kind == GGKS_KIND_TOPK, n, sh.csz, nq)) s.flags |= SEG_SPEC;
   return s;
 }
 
@@ -347,7 +411,8 @@ inline void plan_single(Plan& p, int kind, int dtype, uint64_t n, uint32_t nq,
     }
     for (uint32_t i = 0; i < sh.nitems; ++i)
       p.items.push_back({0u, (uint16_t)(i << sh.gl), (uint16_t)sh.gl});
-    for (uint32_t y = 0; y < ns / kThreads; ++y) p.sblocks.push_back({0u, y});
+    if (!sh.small)
+      for (uint32_t y = 0; y < ns / kThreads; ++y) p.sblocks.push_back({0u, y});
   }
   if (seg_level2(o, sh.mode)) {
     const uint64_t hm = seg_heavy_max(n, nq);
@@ -370,6 +435,14 @@ inline void plan_single(Plan& p, int kind, int dtype, uint64_t n, uint32_t nq,
   p.off_tables = off;
   p.off_segs = take(sizeof(SegDesc));
   p.off_chunks = take((size_t)G * sizeof(Chunk));
+  if (sh.small) {
+    p.small = true;
+    p.nitems = p.nsblocks = 0;
+    p.tables_end = off;
+    layout_small(p, take, 1, (uint64_t)1 << pb, bmax, (bmax + 31) / 32, nq, n, eb);
+    p.total = off;
+    return;
+  }
   p.off_items = take((size_t)sh.nitems * sizeof(ReduceItem));
   p.off_sblocks = take((size_t)(ns / kThreads) * sizeof(SampleBlock));
   p.tables_end = off;
@@ -474,13 +547,34 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
   // 64-bit running totals of the 32-bit offsets, checked before each use
   uint64_t qoff = 0, sam = 0, lutc = 0, totc = 0, bitc = 0, dq = 0;
   uint64_t hmax = 0, cmax = 0;  // second-level capacity
+  // short segments only (k_front / k_back)?
+  auto is_direct = [&](uint64_t n) { return n <= cap && (tab.t[dtype][band_of(n)].direct || n <= 64); };
+  auto bucket_log2 = [&](const BandTuning& bt) {
+    const uint32_t b = o.buckets_log2 ? (uint32_t)o.buckets_log2 : (bt.buckets_log2 ? bt.buckets_log2 : 12u);
+    return std::min<uint32_t>(15, std::max<uint32_t>(8, b));
+  };
+  {
+    uint64_t chunks = 0;
+    p.small = o.level2 <= 0;
+    for (const BatchSeg& g : in) {
+      if (g.num_k == 0 || is_direct(g.length)) continue;
+      if (g.kind == GGKS_KIND_RADIX || !small_len(g.length, eb) || g.num_k > kSmallMaxRanks ||
+          bucket_log2(tab.t[dtype][band_of(g.length)]) > kSmallBucketBits) {
+        p.small = false;
+        break;
+      }
+      const uint64_t c = small_chunk(g.length, eb);
+      chunks += (g.length + c - 1) / c;
+    }
+    if (chunks == 0 || chunks > kSmallMaxChunks) p.small = false;
+  }
   for (size_t i = 0; i < in.size(); ++i) {
     const BatchSeg& g = in[i];
     if (g.num_k == 0) continue;
     const uint64_t n = g.length;
     const BandTuning bt = tab.t[dtype][band_of(n)];
     const bool topk = g.kind == GGKS_KIND_TOPK;
-    if (n <= cap && (bt.direct || n <= 64)) {
+    if (is_direct(n)) {
       if (dq + g.num_k > kPlanTableLimit || p.direct_children.size() >= kPlanGridLimit)
         return false;
       Child c = {};
@@ -511,10 +605,9 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     }
     const bool refine = seg_refine(o, mode);
     if (mode == MODE_SAMPLE || (refine && !o.radix_bits)) {
-      bl = o.buckets_log2 && mode == MODE_SAMPLE ? (uint32_t)o.buckets_log2
-                                                 : (bt.buckets_log2 ? bt.buckets_log2 : 12u);
+      bl = mode == MODE_SAMPLE ? bucket_log2(bt) : bt.buckets_log2 ? bt.buckets_log2 : 12u;
       bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
-      pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
+      pb = p.small ? small_lut_bits(bl) : std::min<uint32_t>(kMaxPrefixBits, bl - 2);
       rb = std::min<uint32_t>(rb, bl - 1);
     }
     const uint32_t bmax = 1u << bl;
@@ -523,6 +616,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     G = std::max<uint64_t>(1, std::min<uint64_t>(G, kMaxChunks));
     csz = (n + G - 1) / G;
     csz = (csz + 63) / 64 * 64;
+    if (p.small) csz = small_chunk(n, eb);
     G = (n + csz - 1) / csz;
     uint32_t ns = 0;
     // one sample per 1024 keys, 1024 to 65536: every sample is a random
@@ -531,7 +625,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     // even, which costs less than the gathers save
     {  // both modes sample: the LUT (bucket) or the digit window (radix)
       uint64_t want = (n / 1024 + 1023) / 1024 * 1024;
-      ns = (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(1024, want));
+      ns = p.small ? small_samples(n, g.num_k, eb) : (uint32_t)std::min<uint64_t>(65536, std::max<uint64_t>(1024, want));
     }
     // every 32-bit offset this segment would take, and the grids, must fit
     const uint32_t nitems = (((bmax + kReduceBins - 1) / kReduceBins) >> reduce_groups_log2(G)) + 1;
@@ -541,7 +635,8 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
         p.chunks.size() + G > kPlanGridLimit || p.items.size() + nitems > kPlanGridLimit ||
         p.sblocks.size() + ns / kThreads > kPlanGridLimit)
       return false;
-    for (uint32_t y = 0; y < ns / kThreads; ++y) p.sblocks.push_back({(uint32_t)p.segs.size(), y});
+    if (!p.small)
+      for (uint32_t y = 0; y < ns / kThreads; ++y) p.sblocks.push_back({(uint32_t)p.segs.size(), y});
     SegDesc s = {};
     s.data_off = g.offset;
     s.len = n;
@@ -563,7 +658,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     s.qsrc = topk ? QSRC_TOPK : QSRC_K;
     s.out_off = (uint32_t)g.out_offset;
     s.flags = refine ? SEG_REFINE : 0u;
-    if (seg_spec(mode == MODE_SAMPLE || refine, topk, n, csz, g.num_k)) s.flags |= SEG_SPEC;
+    if (!p.small && seg_spec(mode == MODE_SAMPLE || refine, topk, n, csz, g.num_k)) s.flags |= SEG_SPEC;
     if (seg_level2(o, mode)) {
       const uint64_t hm = seg_heavy_max(n, g.num_k);
       if (hm > 0) {
@@ -633,6 +728,11 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
   p.off_dchildren = take(p.direct_children.size() * sizeof(Child));
   p.off_dqueries = take(p.direct_queries.size() * sizeof(Query));
   p.tables_end = off;
+  if (p.small) {
+    layout_small(p, take, nseg, lutc, totc, bitc, qoff, red, eb);
+    p.total = off;
+    return true;
+  }
   p.off_states = take(nseg * sizeof(SegState));
   p.off_samples = take((size_t)std::max<uint64_t>(sam, 1) * eb);
   p.off_minmax = take((size_t)std::max<uint64_t>(sam / 1024, 1) * 4 * eb);

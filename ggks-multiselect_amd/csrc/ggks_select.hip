@@ -241,6 +241,11 @@ struct Exec {
   // sampled segment (k_sample counts the sample into it, k_lut reads it and
   // clears it again), owned by the context
   uint32_t* hgram = nullptr;
+  // optional: the call's k list in pinned host memory, copied to k_dst by the
+  // first kernel
+  const uint32_t* hk = nullptr;
+  uint32_t* k_dst = nullptr;
+  uint32_t nk = 0;
 };
 
 static void stage(const Exec& x, int st) {
@@ -278,7 +283,8 @@ static void level_attrs(const Plan&) {
 template <typename KT, int C>
 static void finish(hipStream_t s, const KT* d_src, const KT* red, const KT* red2,
                    const Child* kids, uint32_t n, const Query* cq, const Query* cq2, KT* d_out,
-                   uint32_t max_groups, bool lite, bool small, bool big, const uint32_t* bigw) {
+                   uint32_t max_groups, bool lite, bool small, bool big, const uint32_t* bigw,
+                   uint32_t* zero = nullptr, uint32_t nzero = 0) {
   bool launched = !small;  // small = false: no child for the 256-thread finisher
   if constexpr (sizeof(KT) == 4) {
     if (lite) {
@@ -294,7 +300,7 @@ static void finish(hipStream_t s, const KT* d_src, const KT* red, const KT* red2
   // count of them, read by k_finish before anything else
   if (big)
     hipLaunchKernelGGL((k_finish<KT, C>), dim3(std::min<uint32_t>(n, max_groups)), dim3(kThreads),
-                       kFinishLdsTotal, s, d_src, red, red2, kids, n, cq, cq2, d_out, bigw);
+                       kFinishLdsTotal, s, d_src, red, red2, kids, n, cq, cq2, d_out, bigw, zero, nzero);
 }
 
 // Grid of the second-level kernels (they walk the chunk table with a grid
@@ -332,7 +338,40 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
                   (const Query*)nullptr, d_out, 256, dlite, dsmall, dbig, (const uint32_t*)nullptr);
   };
   const uint32_t nseg = p.nsegs;
-  if (nseg > 0) {
+  if (nseg > 0 && p.small) {
+    const SegDesc* segs = reinterpret_cast<const SegDesc*>(A + p.off_segs);
+    SegState* states = reinterpret_cast<SegState*>(A + p.off_states);
+    const Chunk* chunks = reinterpret_cast<const Chunk*>(A + p.off_chunks);
+    uint32_t* lut = reinterpret_cast<uint32_t*>(A + p.off_lut);
+    uint32_t* tot = reinterpret_cast<uint32_t*>(A + p.off_tot);
+    uint32_t* curs = reinterpret_cast<uint32_t*>(A + p.off_curs);
+    uint32_t* bigw = reinterpret_cast<uint32_t*>(A + p.off_big);
+    Child* kids = reinterpret_cast<Child*>(A + p.off_children);
+    Query* cq = reinterpret_cast<Query*>(A + p.off_cq);
+    KT* red = reinterpret_cast<KT*>(A + p.off_red);
+    for (int st = 1; st <= 3; ++st) stage(x, st);
+    launch_stage(x.prof, 3, k_front<KT, C>, dim3(p.nchunks + (x.nk ? 1 : 0)), dim3(kThreads), 0, s,
+                 d_src, segs, chunks, p.nchunks, p.seed, states, lut, tot, curs, bigw, x.hk, x.k_dst,
+                 x.nk);
+    for (int st = 4; st <= 6; ++st) stage(x, st);
+    if (beside) {
+      HIP_TRY(hipEventRecord(x.fork, s));
+      HIP_TRY(hipStreamWaitEvent(x.side, x.fork, 0));
+      finish_direct(x.side);
+      HIP_TRY(hipEventRecord(x.join, x.side));
+    }
+    launch_stage(x.prof, 6, k_back<KT, C>, dim3(p.nchunks + nseg), dim3(kThreads),
+                 (uint32_t)(kSmallBuckets + kSmallPrefixes + 3 * (kSmallBuckets / 32) + 2 * kSmallRanks + 32) * 4,
+                 s, d_src, chunks, p.nchunks, curs, red, segs, states, lut, tot, (const uint32_t*)nullptr,
+                 (const Query*)nullptr, d_k, x.status, reinterpret_cast<uint32_t*>(A + p.off_qb),
+                 reinterpret_cast<uint32_t*>(A + p.off_qr), kids, cq,
+                 reinterpret_cast<uint32_t*>(A + p.off_bits), reinterpret_cast<uint32_t*>(A + p.off_wbase),
+                 d_out, (uint32_t*)nullptr, (Heavy*)nullptr, (Chunk2*)nullptr, 0u, bigw,
+                 reinterpret_cast<uint2*>(A + p.off_cinfo));
+    stage(x, 7);
+    finish<KT, C>(s, d_src, red, (const KT*)nullptr, kids, p.nq, cq, (const Query*)nullptr, d_out, 256,
+                  elite, true, true, bigw, tot, p.ntot);
+  } else if (nseg > 0) {
     const SegDesc* segs = reinterpret_cast<const SegDesc*>(A + p.off_segs);
     SegState* states = reinterpret_cast<SegState*>(A + p.off_states);
     const Chunk* chunks = reinterpret_cast<const Chunk*>(A + p.off_chunks);
@@ -472,6 +511,10 @@ static uint64_t table_signature(const char* p, size_t n, const void* arena) {
   return h;
 }
 
+static void clear_words(hipStream_t s, void* p, uint32_t n) {
+  hipLaunchKernelGGL(k_clear, dim3((n + 255) / 256), dim3(256), 0, s, static_cast<uint32_t*>(p), n);
+}
+
 // -------------------------------------------------------------- one select
 enum class KSource { HOST, DEVICE, TOPK };
 
@@ -524,7 +567,8 @@ static int select_one(ggks_ctx* c, int kind, int dtype, const void* d_vec, int64
   // plan tables: upload only when they differ from what the arena holds
   std::vector<char> tab(tbytes);
   p.write_tables(tab.data());
-  const uint64_t sig = table_signature(tab.data(), tbytes, c->arena);
+  // (equal tables of key types of two widths differ in where the totals lie)
+  const uint64_t sig = table_signature(tab.data(), tbytes, c->arena) ^ p.off_tot;
   const bool up_tab = sig != c->table_sig, up_k = ksrc == KSource::HOST;
   char* pin = nullptr;
   if (up_tab || up_k || host_out) {
@@ -535,6 +579,8 @@ static int select_one(ggks_ctx* c, int kind, int dtype, const void* d_vec, int64
     HIP_TRY(hipMemcpyAsync(c->arena + p.off_tables, pin, tbytes, hipMemcpyHostToDevice,
                            c->stream));
     c->table_sig = sig;
+    if (p.small)  // k_finish leaves the totals clear for the next call
+      clear_words(c->stream, c->arena + p.off_tot, p.ntot);
   }
   const uint32_t nk = (uint32_t)num_k;
   const uint32_t qgrid = (nk + 255) / 256;
@@ -559,6 +605,7 @@ static int select_one(ggks_ctx* c, int kind, int dtype, const void* d_vec, int64
   Exec x = {c->arena, c->stream, c->status, c->prof_cur >= 0 ? c : nullptr};
   x.hgram = c->hgram;
   rc = launch(x, dtype, p, d_vec, d_out, d_k);
+  if (rc) c->table_sig = 0;
   {
     ggks_debug_regions& g = c->dbg;
     g = ggks_debug_regions{};
@@ -701,13 +748,13 @@ struct SinglePlanArgs {
   SegDesc seg;
   Child dchild;
   uint64_t n, csz;
-  uint32_t G, nitems, gl, nsb, direct;
-  uint64_t off_segs, off_chunks, off_items, off_sblocks, off_dchildren, off_status;
+  uint32_t G, nitems, gl, nsb, direct, ntot;
+  uint64_t off_segs, off_chunks, off_items, off_sblocks, off_dchildren, off_status, off_tot;
 };
 
 // Materialise a single-vector plan's tables in device memory (what the
 // context path uploads from pinned memory) and clear the status block.
-// Thread i writes chunk i, reduce item i and sample block i.
+// Thread i writes chunk i, reduce item i and sample block i and clears total i.
 __global__ __launch_bounds__(256) void k_plan_single(char* __restrict__ base, SinglePlanArgs a) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < 64) reinterpret_cast<uint32_t*>(base + a.off_status)[i] = 0u;
@@ -731,6 +778,7 @@ __global__ __launch_bounds__(256) void k_plan_single(char* __restrict__ base, Si
     it.gi_log2 = (uint16_t)a.gl;
     reinterpret_cast<ReduceItem*>(base + a.off_items)[i] = it;
   }
+  if (i < a.ntot) reinterpret_cast<uint32_t*>(base + a.off_tot)[i] = 0u;
   if (i < a.nsb) {
     SampleBlock sb;
     sb.seg = 0;
@@ -777,9 +825,11 @@ static int select_noalloc(int dtype, const void* d_vec, int64_t n, const uint32_
     if (p.level2) a.seg.flags |= SEG_LEVEL2;
     a.csz = sh.csz;
     a.G = (uint32_t)sh.G;
-    a.nitems = sh.nitems;
+    a.nitems = sh.small ? 0u : sh.nitems;
     a.gl = sh.gl;
-    a.nsb = sh.ns / kThreads;
+    a.nsb = sh.small ? 0u : sh.ns / kThreads;
+    a.ntot = p.ntot;
+    a.off_tot = p.off_tot;
   }
   a.off_segs = p.off_segs;
   a.off_chunks = p.off_chunks;
@@ -787,7 +837,7 @@ static int select_noalloc(int dtype, const void* d_vec, int64_t n, const uint32_
   a.off_sblocks = p.off_sblocks;
   a.off_dchildren = p.off_dchildren;
   a.off_status = off_status;
-  const uint32_t nthreads = std::max<uint32_t>(64, std::max(a.G, std::max(a.nitems, a.nsb)));
+  const uint32_t nthreads = std::max({64u, a.G, a.nitems, a.nsb, a.ntot});
   hipLaunchKernelGGL(k_plan_single, dim3((nthreads + 255) / 256), dim3(256), 0, stream, base, a);
   uint32_t* status = reinterpret_cast<uint32_t*>(base + off_status);
   if (p.direct) {

@@ -124,7 +124,9 @@ static int serve_launch(ggks_server* s, ServeSlot& sl, const std::vector<size_t>
   uint32_t* status = reinterpret_cast<uint32_t*>(arena + align_up(p.total));
   void* d_out = arena + align_up(p.total) + 256;
   HIP_TRY(hipMemcpyAsync(arena + p.off_tables, sl.pinned, tb, hipMemcpyHostToDevice, sl.stream));
-  HIP_TRY(hipMemsetAsync(status, 0, 4, sl.stream));
+  // (a plan of short segments has its totals right below the status word)
+  char* const clear0 = p.small ? arena + p.off_tot : (char*)status;
+  clear_words(sl.stream, clear0, (uint32_t)(((char*)status + 4 - clear0) / 4));
   const Exec x = {arena, sl.stream, status, nullptr};
   const uint32_t* d_k = reinterpret_cast<const uint32_t*>(arena + p.off_kvals);
   const void* src = s->resident[dtype];
