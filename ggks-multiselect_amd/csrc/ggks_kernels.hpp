@@ -2172,10 +2172,19 @@ __global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
 #undef GGKS_FINDK_PARAMS
 #undef GGKS_FINDK_ARGS
 
-// Clear n words (a kernel, so that a caller may capture it).
-__global__ __launch_bounds__(256) void k_clear(uint32_t* __restrict__ p, uint32_t n) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0;
+// Copy up to two blocks of words between pinned host and device memory and
+// clear a third (any of them may be empty; they do not overlap).  One launch
+// costs the host 2.5 us; a copy and a fill by the runtime took 17 us of a
+// served batch of one request (the kernel behind the copy waits for the copy
+// engine), the copy back 4.8.
+__global__ __launch_bounds__(256) void k_stage(uint32_t* __restrict__ d0, const uint32_t* __restrict__ s0,
+                                               uint64_t n0, uint32_t* __restrict__ d1,
+                                               const uint32_t* __restrict__ s1, uint64_t n1,
+                                               uint32_t* __restrict__ zero, uint64_t nz) {
+  const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, step = (uint64_t)gridDim.x * 256;
+  for (uint64_t i = t; i < n0; i += step) d0[i] = s0[i];
+  for (uint64_t i = t; i < n1; i += step) d1[i] = s1[i];
+  for (uint64_t i = t; i < nz; i += step) zero[i] = 0;
 }
 
 // Pass 2 (k_compact): stream the chunk once and move the keys of active

@@ -106,6 +106,9 @@ static int ensure_arena(ggks_ctx* c, size_t bytes) {
   return GGKS_OK;
 }
 
+// Kernels read and write pinned buffers in place.
+constexpr unsigned kPinFlags = hipHostMallocMapped | hipHostMallocCoherent;
+
 // Wait until no copy reads the slot, then make it at least `bytes` long.
 static int pin_ready(PinSlot& s, size_t bytes) {
   if (s.busy) {
@@ -120,7 +123,7 @@ static int pin_ready(PinSlot& s, size_t bytes) {
   s.buf = nullptr;
   s.cap = 0;
   const size_t cap = std::max<size_t>(bytes + bytes / 8, 1 << 16);
-  if (hipHostMalloc(&s.buf, cap, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&s.buf, cap, kPinFlags) != hipSuccess) {
     s.buf = nullptr;
     (void)hipGetLastError();
     return fail(GGKS_ENOMEM, "cannot allocate %zu bytes of pinned memory", cap);
@@ -511,9 +514,26 @@ static uint64_t table_signature(const char* p, size_t n, const void* arena) {
   return h;
 }
 
-static void clear_words(hipStream_t s, void* p, uint32_t n) {
-  hipLaunchKernelGGL(k_clear, dim3((n + 255) / 256), dim3(256), 0, s, static_cast<uint32_t*>(p), n);
+// One launch of k_stage; all sizes in bytes, multiples of 4.
+static void stage_copy(hipStream_t s, void* d0, const void* s0, size_t b0, void* d1 = nullptr,
+                       const void* s1 = nullptr, size_t b1 = 0, void* zero = nullptr, size_t bz = 0) {
+  const uint64_t most = std::max<uint64_t>({b0, b1, bz}) / 4;
+  if (most == 0) return;
+  const uint32_t grid = (uint32_t)std::min<uint64_t>((most + 255) / 256, 1024);
+  hipLaunchKernelGGL(k_stage, dim3(grid), dim3(256), 0, s, static_cast<uint32_t*>(d0),
+                     static_cast<const uint32_t*>(s0), b0 / 4, static_cast<uint32_t*>(d1),
+                     static_cast<const uint32_t*>(s1), b1 / 4, static_cast<uint32_t*>(zero), bz / 4);
 }
+static void clear_words(hipStream_t s, void* p, uint32_t n) {
+  stage_copy(s, nullptr, nullptr, 0, nullptr, nullptr, 0, p, (size_t)n * 4);
+}
+
+// Outputs of a host call up to this size are stored to pinned memory by the
+// finishers themselves: 2 us less than the copy up to 16 KB and 10 to 15 from
+// 32 KB on, where the copy takes another engine.  Past 128 KB it depends on
+// the order of the ranks (130000 outputs, 2^20 floats: 768 -> 747 us sorted,
+// 730 -> 804 shuffled, each a store of 4 bytes over the bus).
+constexpr size_t kDirectOutBytes = 1 << 17;
 
 // -------------------------------------------------------------- one select
 enum class KSource { HOST, DEVICE, TOPK };
@@ -574,24 +594,27 @@ static int select_one(ggks_ctx* c, int kind, int dtype, const void* d_vec, int64
   if (up_tab || up_k || host_out) {
     if ((rc = pin_acquire(c, pin_total, &pin))) return rc;
   }
-  if (up_tab) {
-    memcpy(pin, tab.data(), tbytes);
-    HIP_TRY(hipMemcpyAsync(c->arena + p.off_tables, pin, tbytes, hipMemcpyHostToDevice,
-                           c->stream));
-    c->table_sig = sig;
-    if (p.small)  // k_finish leaves the totals clear for the next call
-      clear_words(c->stream, c->arena + p.off_tot, p.ntot);
-  }
+  // the tables and the k list go up in one launch; the kernels that come
+  // first read the list in place where they can
   const uint32_t nk = (uint32_t)num_k;
   const uint32_t qgrid = (nk + 255) / 256;
   const uint32_t* d_k = k;
+  const uint32_t* hk = up_k ? reinterpret_cast<const uint32_t*>(pin + pin_k) : nullptr;
+  const bool k_in_place = up_k && (p.direct || p.small);
+  if (up_tab) memcpy(pin, tab.data(), tbytes);
   if (up_k) {
     memcpy(pin + pin_k, k, (size_t)num_k * 4);
-    HIP_TRY(hipMemcpyAsync(c->arena + off_dk, pin + pin_k, (size_t)num_k * 4,
-                           hipMemcpyHostToDevice, c->stream));
-    d_k = reinterpret_cast<const uint32_t*>(c->arena + off_dk);
+    d_k = p.direct ? hk : reinterpret_cast<const uint32_t*>(c->arena + off_dk);
   }
-  if ((up_tab || up_k) && (rc = pin_mark(c))) return rc;
+  if (up_tab || (up_k && !k_in_place)) {
+    // k_finish leaves a small plan's totals clear for the next call
+    stage_copy(c->stream, c->arena + p.off_tables, pin, up_tab ? tbytes : 0, c->arena + off_dk, hk,
+               up_k && !k_in_place ? (size_t)num_k * 4 : 0, c->arena + p.off_tot,
+               up_tab && p.small ? (size_t)p.ntot * 4 : 0);
+    c->table_sig = sig;
+  }
+  // a call with host outputs waits for the stream before it returns
+  if (!host_out && up_tab && (rc = pin_mark(c))) return rc;
   if (p.direct) {  // the direct path takes explicit Query records
     Query* d_q = reinterpret_cast<Query*>(c->arena + p.off_dqueries);
     if (ksrc == KSource::TOPK)
@@ -601,9 +624,15 @@ static int select_one(ggks_ctx* c, int kind, int dtype, const void* d_vec, int64
       hipLaunchKernelGGL(k_queries, dim3(qgrid), dim3(256), 0, c->stream, d_k, nk, (uint64_t)n,
                          d_q, c->status);
   }
-  void* d_out = host_out ? (void*)(c->arena + off_dout) : out;
+  const bool out_in_place = host_out && (size_t)num_k * eb <= kDirectOutBytes;
+  void* d_out = out_in_place ? (void*)(pin + pin_out) : host_out ? (void*)(c->arena + off_dout) : out;
   Exec x = {c->arena, c->stream, c->status, c->prof_cur >= 0 ? c : nullptr};
   x.hgram = c->hgram;
+  if (up_k && p.small) {
+    x.hk = hk;
+    x.k_dst = reinterpret_cast<uint32_t*>(c->arena + off_dk);
+    x.nk = nk;
+  }
   rc = launch(x, dtype, p, d_vec, d_out, d_k);
   if (rc) c->table_sig = 0;
   {
@@ -633,12 +662,18 @@ static int select_one(ggks_ctx* c, int kind, int dtype, const void* d_vec, int64
   }
   mark(c, GGKS_NSTAGES);
   c->prof_cur = -1;
-  if (rc) return rc;
+  if (rc) {
+    if (host_out) (void)hipStreamSynchronize(c->stream);  // what runs reads and writes pin
+    return rc;
+  }
   if (host_out) {
     // pin_out is disjoint from every host-written staging region
-    HIP_TRY(hipMemcpyAsync(pin + pin_out, d_out, (size_t)num_k * eb, hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    hipError_t e = hipSuccess;
+    if (!out_in_place)
+      e = hipMemcpyAsync(pin + pin_out, d_out, (size_t)num_k * eb, hipMemcpyDeviceToHost, c->stream);
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    HIP_TRY(e);
+    HIP_TRY(es);
     pin_all_free(c);
     memcpy(out, pin + pin_out, (size_t)num_k * eb);
   }

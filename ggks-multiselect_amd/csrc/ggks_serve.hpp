@@ -7,9 +7,10 @@
 // request of the same dtype (up to max_batch), plans them as one batch
 // (plan_batch), and admits the batch if its scratch (tables, bucket rows,
 // reduced buffer, outputs) fits in the free part of the scratch budget --
-// halving the group until it does.  The batch's tables go up from the slot's
-// pinned buffer, the level kernels run on the slot's stream, the outputs come
-// back to the same pinned buffer and an event marks completion.  Up to
+// halving the group until it does.  A kernel copies the batch's tables up from
+// the slot's pinned buffer and clears its status, the level kernels run on the
+// slot's stream, another kernel brings the outputs back to the same pinned
+// buffer and an event marks completion (k_stage).  Up to
 // max_inflight batches run at once on separate streams, so requests that
 // arrive while others are on the GPU are admitted as slots and memory free
 // up.  Polling harvests finished slots (outputs copied to each request's
@@ -112,7 +113,7 @@ static int serve_launch(ggks_server* s, ServeSlot& sl, const std::vector<size_t>
     sl.pinned = nullptr;
     sl.pinned_cap = 0;
     const size_t cap = std::max<size_t>(pin_need + pin_need / 4, 1 << 20);
-    if (hipHostMalloc(&sl.pinned, cap, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&sl.pinned, cap, kPinFlags) != hipSuccess) {
       (void)hipGetLastError();
       sl.pinned = nullptr;
       return fail(GGKS_ENOMEM, "cannot allocate %zu bytes of pinned memory", cap);
@@ -123,10 +124,10 @@ static int serve_launch(ggks_server* s, ServeSlot& sl, const std::vector<size_t>
   char* arena = s->pool + off;
   uint32_t* status = reinterpret_cast<uint32_t*>(arena + align_up(p.total));
   void* d_out = arena + align_up(p.total) + 256;
-  HIP_TRY(hipMemcpyAsync(arena + p.off_tables, sl.pinned, tb, hipMemcpyHostToDevice, sl.stream));
   // (a plan of short segments has its totals right below the status word)
   char* const clear0 = p.small ? arena + p.off_tot : (char*)status;
-  clear_words(sl.stream, clear0, (uint32_t)(((char*)status + 4 - clear0) / 4));
+  stage_copy(sl.stream, arena + p.off_tables, sl.pinned, tb, nullptr, nullptr, 0, clear0,
+             (size_t)((char*)status + 4 - clear0));
   const Exec x = {arena, sl.stream, status, nullptr};
   const uint32_t* d_k = reinterpret_cast<const uint32_t*>(arena + p.off_kvals);
   const void* src = s->resident[dtype];
@@ -138,8 +139,8 @@ static int serve_launch(ggks_server* s, ServeSlot& sl, const std::vector<size_t>
     default: rc = serve_enqueue_typed<uint32_t, CONV_I>(x, p, src, d_out, d_k); break;
   }
   if (rc) return rc;
-  HIP_TRY(hipMemcpyAsync(sl.pinned + pin_stat, status, 256 + (size_t)outs * eb,
-                         hipMemcpyDeviceToHost, sl.stream));
+  stage_copy(sl.stream, sl.pinned + pin_stat, status, 256 + (size_t)outs * eb);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(sl.done, sl.stream));
   sl.busy = true;
   sl.off = off;
