@@ -1823,7 +1823,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
 
 // ------------------------------------------------------- short segments
 // Plans whose segments are all short (less than 16 MiB of keys, at most 4096
-// buckets and 1024 ranks; Plan::small) run two kernels in place of k_sample,
+// buckets and 8192 ranks; Plan::small) run two kernels in place of k_sample,
 // k_lut, k_count, k_reduce, k_findk and k_compact.  Such selects are bound by
 // launches and by each kernel's chain of dependent round trips, not by
 // bandwidth, so work-groups repeat what used to be handed from one kernel to
@@ -1836,7 +1836,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
 constexpr int kSmallWords = 4;  // 16-byte words of a chunk per thread
 template <typename KT>
 constexpr uint32_t kSmallChunk = kSmallWords * kThreads * 16 / sizeof(KT);
-constexpr uint32_t kSmallBuckets = 4096, kSmallPrefixes = 2048, kSmallRanks = 1024, kSmallSamples = 4096;
+constexpr uint32_t kSmallBuckets = 4096, kSmallPrefixes = 2048, kSmallSamples = 4096;
 
 // A chunk's keys: 16-byte words in registers, at most one unaligned head and
 // one tail key a thread.
@@ -2082,8 +2082,8 @@ __global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
   uint32_t* bits = lut + kSmallPrefixes;    // active buckets
   uint32_t* wb = bits + kSmallBuckets / 32; // first child of a word
   uint32_t* cstart = wb + kSmallBuckets / 32;  // per child: first place, then this chunk's
-  uint32_t* lcnt = cstart + kSmallRanks;       // per child: this chunk's keys
-  uint32_t* wsum = lcnt + kSmallRanks;         // 17
+  uint32_t* lcnt = cstart + kSmallBuckets;     // per child: this chunk's keys
+  uint32_t* wsum = lcnt + kSmallBuckets;       // 17
   const uint32_t tid = threadIdx.x;
   const Chunk ch = chunks[blockIdx.x];
   const SegDesc sd = segs[ch.seg];
@@ -2095,14 +2095,13 @@ __global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
   ck.load(src + sd.data_off + ch.start, (uint32_t)ch.len);
   for (uint32_t i = tid; i < st.P; i += kThreads) lut[i] = lut_pool[sd.lut_off + i];
   if (tid < kSmallBuckets / 32) bits[tid] = 0;
-  lcnt[tid] = 0;
+  for (uint32_t i = tid; i < min(sd.q_cnt, kSmallBuckets); i += kThreads) lcnt[i] = 0;
   const uint32_t B = st.B;
   uint32_t len;
   const uint32_t e = block_excl_scan(t.x + t.y + t.z + t.w, wsum, len);
   if (tid < nt4)
     reinterpret_cast<uint4*>(pre)[tid] = make_uint4(e, e + t.x, e + t.x + t.y, e + t.x + t.y + t.z);
   __syncthreads();
-  auto count_of = [&](uint32_t b) { return (b + 1 < B ? pre[b + 1] : len) - pre[b]; };
   RangeOf<KT> range;
   range.fn.init(st);
   range.lut = lut;
@@ -2110,10 +2109,11 @@ __global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
   range.P = st.P;
   range.s = st.s;
   range.hb = st.hb;
-  // the active buckets, by findk_segment's rules (no more ranks than threads)
-  if (tid < sd.q_cnt) {
-    uint64_t kk = kfirst < 1 || (uint64_t)kfirst > sd.len ? 1 : kfirst;
-    const uint32_t r1 = (uint32_t)(sd.qsrc == QSRC_K ? sd.len - kk : sd.len - tid - 1);
+  // the active buckets, by findk_segment's rules
+  for (uint32_t i = tid; i < sd.q_cnt; i += kThreads) {
+    uint64_t kk = i == tid ? kfirst : sd.qsrc == QSRC_K ? kraw[sd.q_off + i] : 0;
+    if (kk < 1 || kk > sd.len) kk = 1;
+    const uint32_t r1 = (uint32_t)(sd.qsrc == QSRC_K ? sd.len - kk : sd.len - i - 1);
     uint32_t lo = 0, hi = B - 1;  // largest b with pre[b] <= r1
     while (lo < hi) {
       const uint32_t mid = (lo + hi + 1) >> 1;
@@ -2124,21 +2124,17 @@ __global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
     if (klo != khi) lds_or(bits, lo >> 5, 1u << (lo & 31));
   }
   __syncthreads();
-  const uint32_t nwords = (B + 31) / 32;
-  uint32_t m = 0, csum = 0;
-  if (tid < nwords) {
-    m = bits[tid];
-    for (uint32_t mm = m; mm; mm &= mm - 1) csum += count_of(tid * 32 + __ffs(mm) - 1);
-  }
+  // children in bucket order; a thread's four buckets are those of its counts
   uint32_t U, mtot;
+  const uint32_t m = (bits[tid >> 3] >> ((tid & 7) * 4)) & 15u;
+  const uint32_t cc[4] = {m & 1 ? t.x : 0u, m & 2 ? t.y : 0u, m & 4 ? t.z : 0u, m & 8 ? t.w : 0u};
   uint32_t u0 = block_excl_scan((uint32_t)__popc(m), wsum, U);
-  uint32_t c0 = block_excl_scan(csum, wsum, mtot);
-  if (tid < nwords) {
-    wb[tid] = u0;
-    for (uint32_t mm = m; mm; mm &= mm - 1) {
-      cstart[u0++] = c0;
-      c0 += count_of(tid * 32 + __ffs(mm) - 1);
-    }
+  uint32_t c0 = block_excl_scan(cc[0] + cc[1] + cc[2] + cc[3], wsum, mtot);
+  if ((tid & 7) == 0) wb[tid >> 3] = u0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if ((m >> j) & 1u) cstart[u0++] = c0;
+    c0 += cc[j];
   }
   __syncthreads();
   if (U == 0) return;  // uniform
@@ -2160,7 +2156,8 @@ __global__ __launch_bounds__(kThreads) void k_back(const KT* __restrict__ src,
   const uint32_t bh = take(range.fn(to_key<C>(ck.hk), lut), ck.hh);
   const uint32_t bt = take(range.fn(to_key<C>(ck.tk), lut), ck.ht);
   __syncthreads();
-  if (tid < U && lcnt[tid]) cstart[tid] += atomicAdd(&cursors[sd.q_off + tid], lcnt[tid]);
+  for (uint32_t u = tid; u < U; u += kThreads)
+    if (lcnt[u]) cstart[u] += atomicAdd(&cursors[sd.q_off + u], lcnt[u]);
   __syncthreads();
   KT* const rseg = red + sd.red_base;
 #pragma unroll

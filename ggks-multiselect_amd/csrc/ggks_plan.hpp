@@ -106,15 +106,17 @@ inline uint32_t radix_lut_bits(uint32_t rb) { return std::min<uint32_t>(kMaxPref
 constexpr size_t kLutSplitSegs = 16;
 
 // Plans of short segments (k_front / k_back): less than 16 MiB of keys, at
-// most 12 bucket bits, 1024 ranks and 4096 samples each, 512 chunks in all.
+// most 12 bucket bits, 8192 ranks and 4096 samples each, 512 chunks in all.
 // A stream of selects of 1 / 100 / 1000 ranks, six kernels against two:
 // 65537 floats 44 / 47 / 55 -> 27 / 28 / 35 us, 2^20 doubles 51 / 54 / 73 ->
 // 30 / 34 / 40, 3e6 ints 50 / 51 / 63 -> 33 / 42 / 52; where every chunk's
 // work-group's own sample and scans come near what they save, at 4.1e6
 // doubles 68 / 72 / 127 -> 51 / 59 / 71 and 4.1e6 ints 53 / 55 / 72 ->
 // 39 / 48 / 59, the longer pipeline's candidates and wider tables start.
+// Many ranks gain as much: 4000 of 70000 ints 82 -> 54, 8000 of 3e6 floats
+// 238 -> 127, the top 4096 of 7e5 floats 62 -> 53.
 constexpr uint64_t kSmallBytes = 1ull << 24;
-constexpr uint32_t kSmallBucketBits = 12, kSmallMaxRanks = 1024;
+constexpr uint32_t kSmallBucketBits = 12, kSmallMaxRanks = 8192;
 constexpr uint64_t kSmallMaxChunks = 512;
 inline bool small_len(uint64_t n, int eb) { return n * (uint32_t)eb < kSmallBytes; }
 inline uint64_t small_chunk_keys(int eb) { return 4ull * kThreads * 16 / (uint32_t)eb; }

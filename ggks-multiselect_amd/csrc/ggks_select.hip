@@ -364,7 +364,7 @@ static int enqueue_level(const Exec& x, const Plan& p, const KT* d_src, KT* d_ou
       HIP_TRY(hipEventRecord(x.join, x.side));
     }
     launch_stage(x.prof, 6, k_back<KT, C>, dim3(p.nchunks + nseg), dim3(kThreads),
-                 (uint32_t)(kSmallBuckets + kSmallPrefixes + 3 * (kSmallBuckets / 32) + 2 * kSmallRanks + 32) * 4,
+                 (uint32_t)(kSmallBuckets + kSmallPrefixes + 2 * (kSmallBuckets / 32) + 2 * kSmallBuckets + 32) * 4,
                  s, d_src, chunks, p.nchunks, curs, red, segs, states, lut, tot, (const uint32_t*)nullptr,
                  (const Query*)nullptr, d_k, x.status, reinterpret_cast<uint32_t*>(A + p.off_qb),
                  reinterpret_cast<uint32_t*>(A + p.off_qr), kids, cq,

@@ -31,7 +31,7 @@ def test_candidates(pkg, O, dtype, fam):
     W = pkg.workloads
     lib = pkg._lib.lib()
     read_them = 0
-    for n in (MIN - 1, MIN, MIN + 1, (1 << 21) + 5):
+    for n in (MIN - 1, MIN, MIN + 1, (1 << 21) + 5, (1 << 22) + 5):
         x = _x(W, dtype, fam, n)
         d = pkg.DeviceArray.from_host(x)
         m = n // 2

@@ -84,3 +84,23 @@ def test_short_batch(pkg, O):
         print(f"short batch graph={graph}", flush=True)
         assert np.array_equal(bits(b(d, graph=graph)), bits(want))
     b.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32])
+@pytest.mark.parametrize("fam", ["spread", "copies", "heavy"])
+def test_short_many_ranks(pkg, O, dtype, fam):
+    """More ranks than a work-group has threads, up to the limit and past it,
+    repeated and out of order."""
+    W = pkg.workloads
+    ctx = pkg.Context(0)
+    rng = np.random.default_rng(8)
+    for n in (17001, 130001, (1 << 24) // np.dtype(dtype).itemsize - 5):
+        x = _x(W, dtype, fam, n)
+        d = pkg.DeviceArray.from_host(x)
+        for nk in (2047, 4096, 8191, 8192, 8193):
+            print(f"short {np.dtype(dtype).name} {fam} n={n} nk={nk}", flush=True)
+            k = rng.integers(1, n + 1, nk).astype(np.uint32)
+            assert np.array_equal(bits(pkg.multiselect(d, k, ctx)), bits(O.sort_choose(x, k)))
+            assert np.array_equal(bits(pkg.topk(d, nk, ctx)), bits(O.topk(x, nk)))
+        d.free()
+    ctx.close()
