@@ -118,6 +118,9 @@ constexpr size_t kLutSplitSegs = 16;
 constexpr uint64_t kSmallBytes = 1ull << 24;
 constexpr uint32_t kSmallBucketBits = 12, kSmallMaxRanks = 8192;
 constexpr uint64_t kSmallMaxChunks = 512;
+// Radix segments among them whose digits are refined anyway are cut by their
+// sample like the others (1e5 floats, 11 ranks: eleven kernels of 51 us, four of 27).
+inline bool short_radix(const ggks_opts& o) { return o.level2 == 0 && !o.radix_bits; }
 inline bool small_len(uint64_t n, int eb) { return n * (uint32_t)eb < kSmallBytes; }
 inline uint64_t small_chunk_keys(int eb) { return 4ull * kThreads * 16 / (uint32_t)eb; }
 // Chunk length of a short segment: 64 chunks of it (128: 1.2 us more at 5e5
@@ -287,9 +290,12 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
     return sh;
   }
   const Tuning t = single_tuning(dtype, n, nq, kind == GGKS_KIND_TOPK);
-  uint32_t bl;
+  uint32_t bl = o.buckets_log2 ? (uint32_t)o.buckets_log2 : t.buckets_log2;
+  bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
+  sh.small = o.level2 <= 0 && o.blocks <= 0 && small_len(n, eb) && bl <= kSmallBucketBits &&
+             nq <= kSmallMaxRanks && (kind != GGKS_KIND_RADIX || short_radix(o));
   sh.mode = MODE_SAMPLE;
-  if (kind == GGKS_KIND_RADIX) {
+  if (kind == GGKS_KIND_RADIX && !sh.small) {
     sh.mode = MODE_RADIX;
     uint32_t rb = o.radix_bits ? (uint32_t)o.radix_bits : 14u;
     sh.rb = std::min<uint32_t>(14, std::max<uint32_t>(4, rb));
@@ -302,8 +308,6 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
       sh.pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
     }
   } else {
-    bl = o.buckets_log2 ? (uint32_t)o.buckets_log2 : t.buckets_log2;
-    bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
     sh.pb = std::min<uint32_t>(kMaxPrefixBits, bl - 2);
   }
   sh.bmax = 1u << bl;
@@ -312,8 +316,6 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
   G = std::min<uint64_t>(G, kMaxChunks);
   uint64_t csz = (n + G - 1) / G;
   csz = (csz + 63) / 64 * 64;
-  sh.small = sh.mode == MODE_SAMPLE && o.level2 <= 0 && o.blocks <= 0 && small_len(n, eb) &&
-             bl <= kSmallBucketBits && nq <= kSmallMaxRanks;
   if (sh.small) {
     csz = small_chunk(n, eb);
     sh.pb = small_lut_bits(bl);
@@ -560,7 +562,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
     p.small = o.level2 <= 0;
     for (const BatchSeg& g : in) {
       if (g.num_k == 0 || is_direct(g.length)) continue;
-      if (g.kind == GGKS_KIND_RADIX || !small_len(g.length, eb) || g.num_k > kSmallMaxRanks ||
+      if ((g.kind == GGKS_KIND_RADIX && !short_radix(o)) || !small_len(g.length, eb) || g.num_k > kSmallMaxRanks ||
           bucket_log2(tab.t[dtype][band_of(g.length)]) > kSmallBucketBits) {
         p.small = false;
         break;
@@ -598,7 +600,7 @@ inline bool plan_batch(Plan& p, int dtype, const std::vector<BatchSeg>& in, cons
       continue;
     }
     uint32_t mode = MODE_SAMPLE, rb = 0, bl, pb;
-    if (g.kind == GGKS_KIND_RADIX) {
+    if (g.kind == GGKS_KIND_RADIX && !p.small) {
       mode = MODE_RADIX;
       rb = o.radix_bits ? (uint32_t)o.radix_bits : 14u;
       rb = std::min<uint32_t>(14, std::max<uint32_t>(4, rb));

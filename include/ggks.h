@@ -61,7 +61,8 @@ typedef struct ggks_opts {
   int32_t destructive;  /* accepted; the input is never modified */
   uint64_t seed;        /* seed of the splitter sample; 0 = fixed default */
   int32_t radix_bits;   /* radix path: digit width per level (4..14); 0 = 14
-                           (with a bucket budget tuned to the length) */
+                           (with a bucket budget tuned to the length; less
+                           than 16 MiB of keys: cut by a sample) */
   int32_t level2;       /* second level for children of more than 2^16 keys
                            (re-bucketed by the whole GPU): 0 = radix plans
                            only, 1 = every plan, -1 = never */

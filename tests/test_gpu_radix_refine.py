@@ -50,3 +50,29 @@ def test_refined_digits(pkg, O, dtype, fam):
         b.close()
         d.free()
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.uint32, np.int32])
+def test_short_radix_and_single_key_digits(pkg, O, dtype):
+    """Radix selects of short vectors (cut by their sample) and of long ones
+    whose sampled window has a digit per key, with a few keys outside it."""
+    W = pkg.workloads
+    ctx = pkg.Context(0)
+    eb = np.dtype(dtype).itemsize
+    for n in (16385, 100003, (1 << 24) // eb - 1, (1 << 24) // eb, (1 << 24) // eb + 9):
+        for narrow in (False, True):
+            x = W.uint_range(n % 89, n, 0, 1023 if narrow else 2**32 - 1)
+            x = x.view(dtype) if np.dtype(dtype).kind != "f" and not narrow else x.astype(dtype)
+            if narrow:  # keys that no sample is likely to hold
+                x[[5, n // 2, n - 3]] = np.array([1 << 20, 1500, 2000]).astype(dtype)
+                if dtype != np.uint32:
+                    x[7] = -9
+            d = pkg.DeviceArray.from_host(x)
+            for k in (np.array([1, 2, 3, 4, n // 2, n - 1, n]), np.arange(n // 3, n // 3 + 400)):
+                for opts in ({}, {"seed": 5}, {"level2": -1}, {"level2": 1}, {"radix_bits": 11}):
+                    print(f"radix {np.dtype(dtype).name} n={n} narrow={narrow} nk={k.size} {opts}", flush=True)
+                    kk = k.astype(np.uint32)
+                    got = pkg.multiselect(d, kk, ctx, kind="radix", **opts)
+                    assert np.array_equal(bits(got), bits(O.sort_choose(x, kk)))
+            d.free()
+    ctx.close()
