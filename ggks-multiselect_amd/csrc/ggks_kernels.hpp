@@ -1836,7 +1836,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8))) v
 // buckets (k_back).  A chunk is what a work-group holds in registers, so
 // each pass is one round of loads, and the chunks' counts meet in device-scope
 // atomics instead of rows.  2^20 floats, 101 ranks: six kernels of 39 us in
-// all before, two of 22 us (a synchronous call 78.6 -> 56.6 us).
+// all before, two of 25 us (a synchronous call 78.6 -> 54 us).
 constexpr int kSmallWords = 4;  // 16-byte words of a chunk per thread
 template <typename KT>
 constexpr uint32_t kSmallChunk = kSmallWords * kThreads * 16 / sizeof(KT);
