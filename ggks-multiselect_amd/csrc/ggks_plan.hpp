@@ -83,11 +83,26 @@ inline SingleTuningTable& single_tuning_table() {
   static SingleTuningTable tab;
   return tab;
 }
-inline Tuning single_tuning(int dtype, uint64_t n, uint32_t nq, bool topk) {
+inline Tuning single_tuning(int dtype, uint64_t n, uint32_t nq, bool topk, bool radix) {
   int b = 0;
   while (b < kSingleBands - 1 && (n >> (b + 1))) ++b;
   Tuning t = single_tuning_table().t[dtype][b];
-  if (!t.set) t.buckets_log2 = few_ranks_log2(dtype_bytes(dtype), b, nq, topk, t.buckets_log2);
+  if (!t.set) {
+    t.buckets_log2 = few_ranks_log2(dtype_bytes(dtype), b, nq, topk, t.buckets_log2);
+    // more ranks than a quarter of the buckets: spread over the vector they
+    // make most of it active.  One bit more, from 16 MiB of keys on (1500 /
+    // 4000 ranks of 1.6e7 floats 155 / 426 -> 112 / 161 us, 4000 of 3e7 220 ->
+    // 177, of 3e6 doubles 200 -> 161); clustered ranks pay 0 to 15 us for the
+    // wider rows (1500 of 9e6 floats 66 -> 77, of 1.6e7 81 -> 77).  Not where
+    // clusters would pay most: past 2048 ranks of 2^22 4-byte keys (81 -> 100)
+    // and 4-byte radix selects past 2^24 (2100 ranks of 3e7: clustered 113 ->
+    // 123, spread 160 -> 152).
+    const bool four = dtype_bytes(dtype) == 4;
+    if (!topk && t.buckets_log2 < 15 && n * (uint64_t)dtype_bytes(dtype) >= 1ull << 24 &&
+        (uint64_t)nq * 4 > 1ull << t.buckets_log2 && !(four && b == 22 && nq > 2048) &&
+        !(four && radix && b >= 24))
+      t.buckets_log2++;
+  }
   return t;
 }
 
@@ -289,7 +304,7 @@ inline SingleShape single_shape(int kind, int dtype, uint64_t n, uint32_t nq, co
     sh.direct = true;
     return sh;
   }
-  const Tuning t = single_tuning(dtype, n, nq, kind == GGKS_KIND_TOPK);
+  const Tuning t = single_tuning(dtype, n, nq, kind == GGKS_KIND_TOPK, kind == GGKS_KIND_RADIX);
   uint32_t bl = o.buckets_log2 ? (uint32_t)o.buckets_log2 : t.buckets_log2;
   bl = std::min<uint32_t>(15, std::max<uint32_t>(8, bl));
   sh.small = o.level2 <= 0 && o.blocks <= 0 && small_len(n, eb) && bl <= kSmallBucketBits &&
